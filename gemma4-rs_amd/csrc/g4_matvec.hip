@@ -16,9 +16,10 @@
 // block b: its f16 scale and 32 int8 values against the activation's block b
 // (held in the lane's registers for the whole kernel), 8 v_dot4 steps.  The
 // block products go to a table in LDS that lane r then sums for row r in
-// block order, so the run's sequential sums proceed side by side.  The
-// other formats, which the engine uses only for small tensors or for its
-// comparison numerics, give each lane one row and sum sequentially.
+// block order, so the run's sequential sums proceed side by side.  BF16 and
+// F32 rows, one sum per element, split the loading and the adding over two
+// wavefronts.  Q8_0 against f32 activations, the engine's comparison
+// numerics, gives each lane one row.
 
 #include <algorithm>
 #include <type_traits>
@@ -367,30 +368,162 @@ __device__ inline float round_to_bf16(float value) {
     return __uint_as_float(h << 16);
 }
 
-// matvec_bf16 (matvec.rs:124-130, 178-180): x rounded to bf16, one lane per
-// row, one sequential f32 sum over the row.
-__global__ __launch_bounds__(256) void matvec_bf16_kernel(const unsigned short *__restrict__ w, int64_t rows,
-                                                          int64_t cols, const float *__restrict__ x,
-                                                          float *__restrict__ out) {
-#pragma clang fp contract(off)
-    const int64_t row = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (row >= rows) return;
-    const unsigned short *r = w + row * cols;
-    float sum = -0.0f;
-    for (int64_t i = 0; i < cols; ++i) sum += __uint_as_float((unsigned)r[i] << 16) * round_to_bf16(x[i]);
-    out[row] = sum;
-}
+// A value of a BF16 or F32 row as f32, and the activation it meets
+// (matvec_bf16 rounds x to bf16 first).
+__device__ inline float weight_value(unsigned short w) { return __uint_as_float((unsigned)w << 16); }
+__device__ inline float weight_value(float w) { return w; }
+__device__ inline float activation_value(unsigned short, float x) { return round_to_bf16(x); }
+__device__ inline float activation_value(float, float x) { return x; }
 
-// matvec_f32 (matvec.rs:132-136, 182-184): one lane per row, sequential sum.
-__global__ __launch_bounds__(256) void matvec_f32_kernel(const float *__restrict__ w, int64_t rows, int64_t cols,
-                                                         const float *__restrict__ x, float *__restrict__ out) {
+// Waits for this wavefront's LDS work, then the workgroup barrier; loads in
+// flight stay in flight (__syncthreads would wait for them too).
+__device__ inline void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// matvec_bf16 / matvec_f32 (matvec.rs:124-136, 178-184): every row is one
+// sequential f32 sum of its rounded products, so what bounds a row is its
+// chain of adds (one VALU issue, 4 cycles, per element: 2.6 us for 1536
+// columns), and everything else has to stay off the wavefront that adds.  A
+// workgroup of two wavefronts takes R rows.  The first loads them kDenseCols
+// columns at a time (16 bytes per lane, P chunks in flight in registers) and
+// puts the products into one of two tables in LDS; in the other, lane r of
+// the second adds row r's products in order, four to a 16-byte read.
+// Products past the row's end are -0.0, which every sum keeps.  8960 x 1536
+// (weights from HBM) takes 9.9 us in bf16 and 13.9 in f32, against 213 us in
+// bf16 with one lane walking each row in memory (its loads are a row apart)
+// and 14.0 / 14.7 us with one wavefront doing both parts.
+// VEC: rows are read with 16-byte loads through buffer resources: whole loads
+// per row, a matrix on a 4-byte boundary and offsets below 2^31; otherwise
+// value by value.
+constexpr int kDenseCols = 256;
+
+template <typename W, int R, int P, bool VEC>
+__global__ __launch_bounds__(128) void matvec_dense_kernel(const W *__restrict__ w, int64_t rows, int64_t cols,
+                                                           const float *__restrict__ x, float *__restrict__ out) {
 #pragma clang fp contract(off)
-    const int64_t row = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (row >= rows) return;
-    const float *r = w + row * cols;
+    constexpr int E = 16 / sizeof(W);    // values per load
+    constexpr int LPR = kDenseCols / E;  // lanes per row and chunk
+    constexpr int RPI = 64 / LPR;        // rows per load
+    constexpr int NLD = R / RPI;
+    constexpr int TS = kDenseCols + 4;   // table row stride: rows 4 banks apart
+    static_assert(R % RPI == 0 && R <= 64, "whole loads; a lane per row");
+    __shared__ f32x4 table[2][R * TS / 4];
+    const int lane = threadIdx.x & 63;
+    const int64_t row0 = (int64_t)blockIdx.x * R;
+    const int n_rows = (int)min((int64_t)R, rows - row0);
+    const int chunks = (int)((cols + kDenseCols - 1) / kDenseCols);
+
+    if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) == 0) {  // the products
+        const int sub = lane / LPR, g = lane % LPR;
+        const W *base = w + row0 * cols;
+        const uint32_t row_bytes = (uint32_t)(cols * sizeof(W));  // VEC: R * row_bytes < 2^31
+        const __amdgpu_buffer_rsrc_t ws =
+            __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, n_rows * row_bytes, kBufferWord3);
+        const __amdgpu_buffer_rsrc_t xs =
+            __builtin_amdgcn_make_buffer_rsrc((void *)x, 0, (int)(cols * sizeof(float)), kBufferWord3);
+        u32x4 wb[P][NLD];
+        f32x4 xb[P][E / 4];
+        // Chunk c of the rows and of x.  Loads past the last row's end read
+        // zeros, past another's end the next row: the column test replaces
+        // their products.
+        auto load = [&](int c, u32x4 (&wv)[NLD], f32x4 (&xv)[E / 4]) {
+            const int64_t col = (int64_t)c * kDenseCols + E * g;
+            if constexpr (VEC) {
+#pragma unroll
+                for (int j = 0; j < E / 4; ++j)
+                    xv[j] = __builtin_bit_cast(
+                        f32x4, __builtin_amdgcn_raw_buffer_load_b128(xs, (uint32_t)(col + 4 * j) * 4u, 0, 0));
+#pragma unroll
+                for (int j = 0; j < NLD; ++j)
+                    wv[j] = __builtin_amdgcn_raw_buffer_load_b128(
+                        ws, (uint32_t)(j * RPI + sub) * row_bytes + (uint32_t)col * (uint32_t)sizeof(W), 0, 0);
+            } else {
+#pragma unroll
+                for (int j = 0; j < E / 4; ++j)
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) xv[j][k] = col + 4 * j + k < cols ? x[col + 4 * j + k] : 0.0f;
+#pragma unroll
+                for (int j = 0; j < NLD; ++j) {
+                    W v[E];
+                    const int r = j * RPI + sub;
+#pragma unroll
+                    for (int e = 0; e < E; ++e)
+                        v[e] = r < n_rows && col + e < cols ? base[r * cols + col + e] : (W)0;
+                    wv[j] = __builtin_bit_cast(u32x4, v);
+                }
+            }
+        };
+        auto products = [&](int c, const u32x4 (&wv)[NLD], const f32x4 (&xv)[E / 4], auto whole) {
+            float xa[E];
+#pragma unroll
+            for (int e = 0; e < E; ++e) xa[e] = activation_value(W(), xv[e / 4][e % 4]);
+            float *t = (float *)table[c & 1] + sub * TS + E * g;
+#pragma unroll
+            for (int j = 0; j < NLD; ++j) {
+                W v[E];
+                __builtin_memcpy(v, &wv[j], 16);
+#pragma unroll
+                for (int q = 0; q < E / 4; ++q) {
+                    f32x4 pr;
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        const int e = 4 * q + k;
+                        pr[k] = weight_value(v[e]) * xa[e];
+                        if (!decltype(whole)::value && (int64_t)c * kDenseCols + E * g + e >= cols) pr[k] = -0.0f;
+                    }
+                    *(f32x4 *)(t + j * RPI * TS + 4 * q) = pr;
+                }
+            }
+        };
+#pragma unroll
+        for (int p = 0; p < P; ++p) load(p, wb[p], xb[p]);
+        for (int c0 = 0; c0 < chunks; c0 += P) {
+#pragma unroll
+            for (int p = 0; p < P; ++p) {
+                const int c = c0 + p;
+                if (c >= chunks) break;
+                if ((int64_t)(c + 1) * kDenseCols <= cols)
+                    products(c, wb[p], xb[p], std::true_type());
+                else
+                    products(c, wb[p], xb[p], std::false_type());
+                load(c + P, wb[p], xb[p]);
+                lds_barrier();  // chunk c is in its table; chunk c - 1 has been added
+            }
+        }
+        return;
+    }
     float sum = -0.0f;
-    for (int64_t i = 0; i < cols; ++i) sum += r[i] * x[i];
-    out[row] = sum;
+    for (int c = 0; c < chunks; ++c) {
+        lds_barrier();
+        const f32x4 *tr = table[c & 1] + (lane % R) * (TS / 4);
+        const int n = (int)min((int64_t)kDenseCols, cols - (int64_t)c * kDenseCols);
+        // 32 products read ahead of the 32 being added.
+        f32x4 a[8], b[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) a[i] = tr[i];
+#pragma unroll
+        for (int s = 0; s < kDenseCols / 32; s += 2) {
+            if (32 * s >= n) break;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) b[i] = tr[8 * (s + 1) + i];
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+#pragma unroll
+                for (int k = 0; k < 4; ++k) sum += a[i][k];
+            __builtin_amdgcn_sched_barrier(0);
+            if (s + 2 < kDenseCols / 32) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) a[i] = tr[8 * (s + 2) + i];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+#pragma unroll
+                for (int k = 0; k < 4; ++k) sum += b[i][k];
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    if (lane < n_rows) out[row0 + lane] = sum;
 }
 
 template <int EPI, int NS, bool STREAM>
@@ -471,6 +604,27 @@ int launch_q8(g4_ctx *ctx, MatvecArgs a, hipStream_t stream) {
     return G4_OK;
 }
 
+template <typename W, int R, int P, bool VEC>
+int launch_dense_rows(const MatvecArgs &a, hipStream_t stream) {
+    hipLaunchKernelGGL((matvec_dense_kernel<W, R, P, VEC>), dim3((unsigned)((a.rows + R - 1) / R)), dim3(128), 0,
+                       stream, (const W *)a.w, a.rows, a.cols, a.x, a.out);
+    G4_HIP(hipGetLastError());
+    return G4_OK;
+}
+
+// Rows per workgroup of the BF16 / F32 mat-vecs.  Up to eight rows per CU
+// every wavefront has a SIMD of its own with 4 rows, and the shorter loads
+// start the chain sooner (1024 x 1536 bf16: 6.6 us against 7.2 with 16).
+// Beyond that the adding wavefronts share SIMDs, and an add costs the same
+// for 4 rows as for 16 (8960 x 1536: 14.3 us with 4, 11.3 with 8, 9.9 with 16).
+template <typename W>
+int launch_dense(g4_ctx *ctx, const MatvecArgs &a, hipStream_t stream) {
+    const bool vec = (uintptr_t)a.w % 4 == 0 && a.cols * sizeof(W) % 16 == 0 && a.cols < (1LL << 24);
+    if (!vec) return launch_dense_rows<W, 4, 2, false>(a, stream);
+    if (a.rows <= 8LL * ctx->num_cus) return launch_dense_rows<W, 4, 4, true>(a, stream);
+    return launch_dense_rows<W, 16, 3, true>(a, stream);
+}
+
 }  // namespace
 
 int launch_quantize_q8_0(const float *x, int64_t n, float *scales, signed char *quants, hipStream_t stream) {
@@ -497,14 +651,8 @@ int launch_matvec(g4_ctx *ctx, const MatvecArgs &a, hipStream_t stream) {
         hipLaunchKernelGGL(matvec_q8_0_f32_kernel<true>, dim3(grid), dim3(256), 0, stream, a.w, a.rows,
                            (int)(a.cols / kQ8Values), a.x, a.out);
         break;
-    case MatvecKind::Bf16:
-        hipLaunchKernelGGL(matvec_bf16_kernel, dim3(grid), dim3(256), 0, stream, (const unsigned short *)a.w, a.rows,
-                           a.cols, a.x, a.out);
-        break;
-    case MatvecKind::F32:
-        hipLaunchKernelGGL(matvec_f32_kernel, dim3(grid), dim3(256), 0, stream, (const float *)a.w, a.rows, a.cols,
-                           a.x, a.out);
-        break;
+    case MatvecKind::Bf16: return launch_dense<unsigned short>(ctx, a, stream);
+    case MatvecKind::F32: return launch_dense<float>(ctx, a, stream);
     }
     G4_HIP(hipGetLastError());
     return G4_OK;

@@ -148,6 +148,31 @@ def test_bf16_and_f32_matvecs_bit_exact(ctx, rows, cols):
     assert np.array_equal(host(out).view(np.uint32), orc.matvec_bf16(wb, rows, cols, x).view(np.uint32))
 
 
+@pytest.mark.parametrize("rows,cols", [(1, 1), (3, 8), (4, 255), (5, 256), (15, 257), (16, 264), (2048, 520), (2049, 520),
+                                       (2065, 1032), (2064, 250), (6, 40000)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_bf16_and_f32_matvecs_at_the_tiles_edges(ctx, rows, cols, shift):
+    """Row and column counts around the workgroup's rows and chunks, matrices
+    off a 4-byte boundary (shift, in values), and rows holding inf, NaN and
+    only zero products of either sign, whose sums' bits are the oracle's."""
+    print(f"[case] dense {rows}x{cols} shift {shift}", flush=True)
+    rng = np.random.default_rng(rows + cols)
+    w = rng.standard_normal(rows * cols).astype(np.float32).reshape(rows, cols)
+    x = rng.standard_normal(cols).astype(np.float32)
+    w[0] = -0.0 * np.sign(x)  # every product -0.0 or +0.0
+    w[rows // 2, cols // 2] = np.inf
+    w[rows - 1, cols - 1] = -1e30
+    wb = ((w.view(np.uint32) + 0x7FFF + ((w.view(np.uint32) >> 16) & 1)) >> 16).astype(np.uint16)
+    for call, ref_of, m in ((ctx.matvec_f32, orc.matvec_f32, w), (ctx.matvec_bf16, orc.matvec_bf16, wb)):
+        out = torch.full((rows + 1,), 7.0, device="cuda")
+        d = dev(np.concatenate([np.zeros(shift, m.dtype), m.reshape(-1)]))[shift:]
+        call(d, rows, cols, dev(x), out)
+        got, ref = host(out), ref_of(m.reshape(-1), rows, cols, x)
+        assert got[rows] == 7.0
+        same = (got[:rows].view(np.uint32) == ref.view(np.uint32)) | (np.isnan(got[:rows]) & np.isnan(ref))
+        assert same.all(), np.flatnonzero(~same)[:8]
+
+
 def test_bf16_known_answer(ctx):
     """tests/matvec.rs:109-120: x is rounded to bf16 before the product."""
     w = np.array([orc.f32_to_bf16(2.0), orc.f32_to_bf16(-0.5)], np.uint16)
