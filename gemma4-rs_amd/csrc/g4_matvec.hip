@@ -16,10 +16,11 @@
 // block b: its f16 scale and 32 int8 values against the activation's block b
 // (held in the lane's registers for the whole kernel), 8 v_dot4 steps.  The
 // block products go to a table in LDS that lane r then sums for row r in
-// block order, so the run's sequential sums proceed side by side.  BF16 and
-// F32 rows, one sum per element, split the loading and the adding over two
-// wavefronts.  Q8_0 against f32 activations, the engine's comparison
-// numerics, gives each lane one row.
+// block order, so the run's sequential sums proceed side by side.  Matrices
+// below the output head's size bring all their rows at once instead, with the
+// activation quantized once per workgroup (f32 activations, the engine's
+// comparison numerics, go the same way).  BF16 and F32 rows, one sum per
+// element, split the loading and the adding over two wavefronts.
 
 #include <algorithm>
 #include <type_traits>
@@ -105,39 +106,6 @@ __global__ __launch_bounds__(256) void quantize_q8_0_kernel(const float *x, int6
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-// One block of 32 activation values (block b of x, 16-byte aligned).
-__device__ inline void load_block(const float *x, int b, f32x4 (&v)[8]) {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = ((const f32x4 *)(x + kQ8Values * b))[j];
-}
-
-// One lane's quantize_q8_0 of a loaded block: the same arithmetic as
-// quantize_q8_0_kernel, the 32 values packed 4 to a dword.
-__device__ inline float quantize_values(const f32x4 (&v)[8], int (&q)[8]) {
-#pragma clang fp contract(off)
-    float m = 0.0f;
-#pragma unroll
-    for (int j = 0; j < 8; ++j)
-#pragma unroll
-        for (int k = 0; k < 4; ++k) m = fmaxf(m, fabsf(v[j][k]));
-    const float scale = m / 127.0f;
-    const float inverse = scale == 0.0f ? 0.0f : 1.0f / scale;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        unsigned packed = 0;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) packed |= ((unsigned)saturate_i8(rintf(v[j][k] * inverse)) & 0xffu) << (8 * k);
-        q[j] = (int)packed;
-    }
-    return round_to_half(scale);
-}
-
-__device__ inline float quantize_block(const float *x, int b, int (&q)[8]) {
-    f32x4 v[8];
-    load_block(x, b, v);
-    return quantize_values(v, q);
-}
-
 // Epilogues of the Q8_0 row kernel.
 enum Epilogue : int { kPlain = 0, kSoftcap = 1, kGeglu = 2, kGegluFp16 = 3 };
 
@@ -148,15 +116,15 @@ enum Epilogue : int { kPlain = 0, kSoftcap = 1, kGeglu = 2, kGegluFp16 = 3 };
 // 64 s) into a row-major product table in LDS; once all rows are done, lane
 // r sums row r's products in block order -- up to 64 independent sequential
 // sums at once, each exactly the reference's.  kGeglu* read a second matrix
-// (up) beside the first (gate).  Large matrices stage one row at a time in
-// small workgroups, so that many are resident per CU (measured faster than
-// double-buffering fewer of them); small ones stage all their rows at once.
-template <int EPI, int NS, bool STREAM>
+// (up) beside the first (gate).  For large matrices: small workgroups, so
+// that many are resident per CU (measured faster than double-buffering fewer
+// of them).
+template <int EPI, int NS>
 __global__ __launch_bounds__(64) void matvec_q8_0_kernel(const unsigned char *__restrict__ w,
                                                          const unsigned char *__restrict__ w2, int64_t rows,
                                                          int nb, const float *__restrict__ xs,
-                                                         const int *__restrict__ xq, const float *__restrict__ xf,
-                                                         float arg, int g, int rb, float *__restrict__ out) {
+                                                         const int *__restrict__ xq, float arg, int g, int rb,
+                                                         float *__restrict__ out) {
 #pragma clang fp contract(off)
     extern __shared__ u32x4 lds[];
     constexpr int NM = EPI >= kGeglu ? 2 : 1;  // matrices read
@@ -180,47 +148,20 @@ __global__ __launch_bounds__(64) void matvec_q8_0_kernel(const unsigned char *__
                 u32x4 *dst = stage + (r * NM + m) * chunks;
                 for (int k = 0; k * 64 < chunks; ++k)
                     if (k * 64 + lane < chunks)
-                        load_to_lds<STREAM ? kNonTemporal : 0>(rs, dst + 64 * k, (uint32_t)(k * 64 + lane) * 16u);
+                        load_to_lds<kNonTemporal>(rs, dst + 64 * k, (uint32_t)(k * 64 + lane) * 16u);
             }
     };
-    // The first rows' loads are in flight while the activation is read (and
-    // quantized, when it comes as f32).  Small matrices quantize the f32
-    // activation here: its loads go first, since load counters complete in
-    // issue order and the quantization would otherwise wait for the rows
-    // (q projection 4096 x 1536: 8.05 -> 7.52 us).  Large ones read a
-    // quantized activation after their rows (the order measured faster).
-    f32x4 xv[STREAM ? 1 : NS][8];
-    if constexpr (!STREAM) {
-        if (xf) {
-#pragma unroll
-            for (int s = 0; s < NS; ++s) load_block(xf, min(lane + 64 * s, nb - 1), xv[s]);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-    }
+    // The first rows' loads are in flight while the activation is read: this
+    // lane's blocks, 8 packed int8 dwords and the scale each.
     stage_rows(0);
-    if constexpr (!STREAM) __builtin_amdgcn_sched_barrier(0);
-
-    // This lane's activation blocks: 8 packed int8 dwords and the scale.
     int xqr[NS][8];
     float xsr[NS];
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
         const int b = lane + 64 * s;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) xqr[s][j] = 0;
-        xsr[s] = 0.0f;
-        if (b < nb) {
-            if (xf) {  // quantize_q8_0 of the f32 activation, here
-                if constexpr (STREAM)
-                    xsr[s] = quantize_block(xf, b, xqr[s]);
-                else
-                    xsr[s] = quantize_values(xv[s], xqr[s]);
-            } else {
-#pragma unroll
-                for (int j = 0; j < 8; ++j) xqr[s][j] = xq[b * 8 + j];
-                xsr[s] = xs[b];
-            }
-        }
+        for (int j = 0; j < 8; ++j) xqr[s][j] = b < nb ? xq[b * 8 + j] : 0;
+        xsr[s] = b < nb ? xs[b] : 0.0f;
     }
 
     for (int r0 = 0; r0 < n_rows; r0 += g) {
@@ -280,6 +221,228 @@ __global__ __launch_bounds__(64) void matvec_q8_0_kernel(const unsigned char *__
     if constexpr (EPI == kGeglu) v = gelu_tanh(acc[0]) * acc[NM - 1];
     if constexpr (EPI == kGegluFp16) v = gelu_tanh_fp16_table(acc[0]) * acc[NM - 1];
     out[row0 + lane] = v;
+}
+
+// LDS of matvec_q8_0_once_kernel, in bytes unless said: the activation, then
+// per row wavefront the rows it brings (per matrix) and its product table.
+struct Q8OnceLds {
+    int padded, pstride;  // products per row: rounded up to 16, and apart
+    int act, stage, wave;
+    __host__ __device__ Q8OnceLds(int nb, int rw, int nm, int value_bytes, int act_block)
+        : padded((nb + 15) / 16 * 16), pstride(padded + 16 / value_bytes), act((nb * act_block * 4 + 15) / 16 * 16),
+          stage((rw * nb * kQ8Bytes + 2 + 15) / 16 * 16), wave(nm * (stage + rw * pstride * value_bytes)) {}
+};
+
+// What a block's product is: the integer dot of quantized activations, or
+// the sequential f32 / f64 sum against f32 activations.
+enum Dot : int { kInt8 = 0, kF32 = 1, kF64 = 2 };
+
+// Largest of v over each run of 8 lanes (NaN ignored, as fmaxf does).
+__device__ inline float max8(float v) {
+    auto from = [](float x, auto ctrl) {
+        return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), decltype(ctrl)::value, 0xf, 0xf, true));
+    };
+    v = fmaxf(v, from(v, std::integral_constant<int, 0xB1>()));  // quad_perm [1,0,3,2]
+    v = fmaxf(v, from(v, std::integral_constant<int, 0x4E>()));  // quad_perm [2,3,0,1]
+    return fmaxf(v, from(v, std::integral_constant<int, 0x141>()));  // row_half_mirror
+}
+
+// Dwords of an activation block in LDS: 8 of int8 values and the scale, or
+// 32 f32 values, padded so that 16-byte reads by consecutive lanes spread
+// over the banks.
+template <int DOT> constexpr int kActBlock = DOT == kInt8 ? 12 : 36;
+
+// The activation into LDS by nq wavefronts (t: thread among them), 8 lanes
+// per block, 6 blocks of a lane group in flight: quantized here when it
+// comes as f32 (the arithmetic of quantize_q8_0_kernel), else copied.
+template <int DOT>
+__device__ inline void stage_activation(float *act, int nb, const float *xs, const int *xq, const float *xf, int t,
+                                        int nq) {
+#pragma clang fp contract(off)
+    const int j = t & 7, step = 8 * nq;
+    if (DOT == kInt8 && xs) {
+        for (int b = t >> 3; b < nb; b += step) {
+            ((int *)act)[b * 12 + j] = xq[b * 8 + j];
+            if (j == 0) act[b * 12 + 8] = xs[b];
+        }
+        return;
+    }
+    constexpr int NF = 6;
+    const bool aligned = ((uintptr_t)xf & 15) == 0;
+    for (int b0 = t >> 3; b0 < nb; b0 += NF * step) {
+        f32x4 v[NF];
+#pragma unroll
+        for (int i = 0; i < NF; ++i) {
+            const float *src = xf + kQ8Values * min(b0 + i * step, nb - 1) + 4 * j;
+            if (aligned)
+                v[i] = *(const f32x4 *)src;
+            else
+                v[i] = f32x4{src[0], src[1], src[2], src[3]};
+        }
+#pragma unroll
+        for (int i = 0; i < NF; ++i) {
+            const int b = b0 + i * step;
+            if (b >= nb) break;
+            if constexpr (DOT == kInt8) {
+                float m = 0.0f;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) m = fmaxf(m, fabsf(v[i][k]));
+                const float scale = max8(m) / 127.0f;
+                const float inverse = scale == 0.0f ? 0.0f : 1.0f / scale;
+                unsigned packed = 0;
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    packed |= ((unsigned)saturate_i8(rintf(v[i][k] * inverse)) & 0xffu) << (8 * k);
+                ((int *)act)[b * 12 + j] = (int)packed;
+                if (j == 0) act[b * 12 + 8] = round_to_half(scale);
+            } else {
+                *(f32x4 *)(act + b * 36 + 4 * j) = v[i];
+            }
+        }
+    }
+}
+
+// W @ x for Q8_0 rows, the matrices that do not fill the chip for long
+// (everything but the output head).  They are bound by one trip to memory,
+// so every byte is asked for at once: about one workgroup per CU, whose nw
+// row wavefronts each bring rw consecutive rows (one run of bytes, per
+// matrix) into LDS with 16-byte direct-to-LDS loads, while nq further
+// wavefronts load the activation, quantize it once for the workgroup and
+// leave it in LDS.  Those are other wavefronts because load counters
+// complete in order: a row wavefront that also read the activation would
+// wait for its rows first.  Then lane b of a row wavefront forms block b's
+// product of each of its rows (b = lane, lane + 64, ...) in a table, and
+// lane r sums row r's products in block order.  Rows need not be 16-byte
+// aligned: a run is loaded from the dword its first byte lies in, its last
+// bytes (fewer than 16) as 2-byte values.
+// Weights from HBM, activation as f32 (one wavefront per two or three rows
+// that quantized the activation for itself, before -> here): 2048 x 1536
+// 5.4 -> 4.0 us, 4096 x 1536 6.3 -> 5.0, 1536 x 6144 11.3 -> 7.5, gate and up
+// of 6144 x 1536 (20.9 MB) 10.3 -> 7.7; a plain read of 16 MiB takes 4.7.
+// f32 activations, one lane per row before: 2048 x 1536 27 -> 3.8 us,
+// 1536 x 6144 172 -> 7.4.
+template <int EPI, int DOT>
+__global__ __launch_bounds__(768) void matvec_q8_0_once_kernel(const unsigned char *__restrict__ w,
+                                                               const unsigned char *__restrict__ w2, int64_t rows,
+                                                               int nb, const float *__restrict__ xs,
+                                                               const int *__restrict__ xq,
+                                                               const float *__restrict__ xf, float arg, int nw, int nq,
+                                                               int rw, float *__restrict__ out) {
+#pragma clang fp contract(off)
+    using T = typename std::conditional<DOT == kF64, double, float>::type;
+    typedef T vec __attribute__((ext_vector_type(16 / sizeof(T))));
+    constexpr int NM = EPI >= kGeglu ? 2 : 1;  // matrices read
+    constexpr int V = 16 / sizeof(T);          // products per 16-byte read
+    extern __shared__ u32x4 lds[];
+    float *act = (float *)lds;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const Q8OnceLds at(nb, rw, NM, (int)sizeof(T), kActBlock<DOT>);
+    if (wave >= nw) {
+        stage_activation<DOT>(act, nb, xs, xq, xf, threadIdx.x - 64 * nw, nq);
+        __syncthreads();
+        return;
+    }
+    unsigned char *mine = (unsigned char *)lds + at.act + (size_t)wave * at.wave;  // this wavefront's rows and products
+    T *prod = (T *)(mine + NM * at.stage);                                         // [NM][rw][pstride]
+    const int row_len = nb * kQ8Bytes;
+    const int64_t row0 = ((int64_t)blockIdx.x * nw + wave) * rw;
+    const int n = (int)max((int64_t)0, min((int64_t)rw, rows - row0));
+    const int64_t first = row0 * row_len;
+    const int skew = (int)(first & 3);  // 0 or 2
+    if (n > 0) {
+        const int bytes = n * row_len + skew, chunks = bytes >> 4, rest = bytes & 15;
+#pragma unroll
+        for (int m = 0; m < NM; ++m) {
+            const unsigned char *src = (m == 0 ? w : w2) + (first - skew);
+            const __amdgpu_buffer_rsrc_t rs =
+                __builtin_amdgcn_make_buffer_rsrc((void *)src, 0, chunks * 16, kBufferWord3);
+            u32x4 *dst = (u32x4 *)(mine + m * at.stage);
+            for (int k = 0; k < chunks; k += 64)
+                if (k + lane < chunks) load_to_lds<0>(rs, dst + k, (uint32_t)(k + lane) * 16u);
+            if (2 * lane < rest)
+                ((unsigned short *)(dst + chunks))[lane] = ((const unsigned short *)(src + chunks * 16))[lane];
+        }
+    }
+    __builtin_amdgcn_s_waitcnt(kVmcntZero);
+    __syncthreads();
+    if (n <= 0) return;
+
+    for (int b = lane; b < at.padded; b += 64) {
+        int xi[8];
+        float xr[DOT == kInt8 ? 1 : kQ8Values];
+        if constexpr (DOT == kInt8) {
+            const int *src = (const int *)act + min(b, nb - 1) * 12;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) xi[j] = src[j];
+            xr[0] = ((const float *)src)[8];
+        } else {
+            const float *src = act + min(b, nb - 1) * 36;
+#pragma unroll
+            for (int j = 0; j < kQ8Values; ++j) xr[j] = src[j];
+        }
+        for (int r = 0; r < n; ++r)
+#pragma unroll
+            for (int m = 0; m < NM; ++m) {
+                T *pr = prod + (m * rw + r) * at.pstride + b;
+                if (b >= nb) {  // every sum keeps -0.0
+                    *pr = (T)-0.0;
+                    continue;
+                }
+                // The block's scale is in its first two bytes, the values
+                // follow: in 9 dwords, one half left over.
+                const int off = skew + r * row_len + kQ8Bytes * b;
+                const unsigned *d = (const unsigned *)(mine + m * at.stage) + (off >> 2);
+                unsigned raw[9], q[8];
+#pragma unroll
+                for (int j = 0; j < 9; ++j) raw[j] = d[j];
+                const bool high = off & 2;
+                const float ws = half_bits_to_float(high ? raw[0] >> 16 : raw[0]);
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    q[j] = high ? raw[j + 1] : __builtin_amdgcn_alignbyte(raw[j + 1], raw[j], 2);
+                if constexpr (DOT == kInt8) {
+                    int dot = 0;
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) dot = __builtin_amdgcn_sdot4((int)q[j], xi[j], dot, false);
+                    *pr = (float)dot * (ws * xr[0]);  // matvec.rs:148
+                } else {  // matvec.rs:153-176: the 32 products in order, then the scale
+                    T dot = (T)-0.0;
+#pragma unroll
+                    for (int j = 0; j < 8; ++j)
+#pragma unroll
+                        for (int k = 0; k < 4; ++k)
+                            dot += (T)(int)(signed char)(q[j] >> (8 * k)) * (T)xr[4 * j + k];
+                    *pr = dot * (T)ws;
+                }
+            }
+    }
+    // Lane m*rw + r sums row r of matrix m, 16 products read ahead.
+    T sum = (T)-0.0;
+    if (lane < NM * rw) {
+        const vec *pr = (const vec *)(prod + lane * at.pstride);
+        vec cur[16 / V], nxt[16 / V];
+#pragma unroll
+        for (int i = 0; i < 16 / V; ++i) cur[i] = pr[i];
+        for (int b = 16; b <= at.padded; b += 16) {
+            const int ahead = min(b, at.padded - 16) / V;
+#pragma unroll
+            for (int i = 0; i < 16 / V; ++i) nxt[i] = pr[ahead + i];
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < 16 / V; ++i)
+#pragma unroll
+                for (int k = 0; k < V; ++k) sum += cur[i][k];
+#pragma unroll
+            for (int i = 0; i < 16 / V; ++i) cur[i] = nxt[i];
+        }
+    }
+    float v = (float)sum;
+    if constexpr (EPI == kSoftcap) v = tanhf(v * (1.0f / arg)) * arg;  // ops.rs:79-81
+    if constexpr (NM == 2) {
+        const float up = __shfl(v, lane + rw);
+        v = (EPI == kGeglu ? gelu_tanh(v) : gelu_tanh_fp16_table(v)) * up;
+    }
+    if (lane < n) out[row0 + lane] = v;
 }
 
 // Reads the 34-byte Q8_0 block at byte `off` of a row (2-byte aligned):
@@ -526,15 +689,52 @@ __global__ __launch_bounds__(128) void matvec_dense_kernel(const W *__restrict__
     if (lane < n_rows) out[row0 + lane] = sum;
 }
 
-template <int EPI, int NS, bool STREAM>
+template <int EPI, int NS>
 int launch_q8_rows(const MatvecArgs &a, int g, int rb, hipStream_t stream) {
     constexpr int NM = EPI >= kGeglu ? 2 : 1;
     const int nb = (int)(a.cols / kQ8Values);
     const size_t lds = (size_t)g * NM * (nb * kQ8Bytes) + (size_t)NM * rb * (nb + 1) * sizeof(float);
     const int64_t groups = (a.rows + rb - 1) / rb;
-    hipLaunchKernelGGL((matvec_q8_0_kernel<EPI, NS, STREAM>), dim3((unsigned)groups), dim3(64), lds, stream, a.w, a.w2,
-                       a.rows, nb, a.xs, (const int *)a.xq, a.xs ? nullptr : a.x, a.arg, g, rb, a.out);
+    hipLaunchKernelGGL((matvec_q8_0_kernel<EPI, NS>), dim3((unsigned)groups), dim3(64), lds, stream, a.w, a.w2, a.rows,
+                       nb, a.xs, (const int *)a.xq, a.arg, g, rb, a.out);
     G4_HIP(hipGetLastError());
+    return G4_OK;
+}
+
+// Launches matvec_q8_0_once_kernel, or says (*done) that the shape does not
+// suit it: a matrix off a 4-byte boundary, no blocks, or rows too long for a
+// CU's LDS.
+template <int EPI, int DOT>
+int launch_q8_once(g4_ctx *ctx, const MatvecArgs &a, hipStream_t stream, bool *done) {
+    constexpr int NM = EPI >= kGeglu ? 2 : 1;
+    constexpr int kValue = DOT == kF64 ? 8 : 4;
+    *done = false;
+    const int64_t nb64 = a.cols / kQ8Values;
+    if (nb64 <= 0 || nb64 > 8192 || (uintptr_t)a.w % 4 != 0 || (NM == 2 && (uintptr_t)a.w2 % 4 != 0)) return G4_OK;
+    const int nb = (int)nb64;
+    // One workgroup per CU with a row wavefront per row, up to 8, then more
+    // rows per wavefront; where that does not fit a CU's LDS, two workgroups
+    // per CU, each within half of it.
+    constexpr size_t kLds = 160 * 1024;
+    auto bytes = [&](int nw, int rw) {
+        const Q8OnceLds at(nb, rw, NM, kValue, kActBlock<DOT>);
+        return (size_t)at.act + (size_t)nw * at.wave;
+    };
+    const int64_t per_cu = std::min<int64_t>(8 * (64 / NM), (a.rows + ctx->num_cus - 1) / ctx->num_cus);
+    int nw = (int)std::min<int64_t>(8, per_cu), rw = (int)((per_cu + nw - 1) / nw);
+    if (bytes(nw, rw) > kLds) {
+        while (rw > 1 && bytes(nw, rw) > kLds / 2) --rw;
+        while (nw > 1 && bytes(nw, rw) > kLds / 2) --nw;
+        if (bytes(nw, rw) > kLds) return G4_OK;
+    }
+    const int nq = std::min(4, (nb + 23) / 24);
+    const int64_t groups = (a.rows + (int64_t)nw * rw - 1) / ((int64_t)nw * rw);
+    if (groups >= (1LL << 31)) return G4_OK;
+    hipLaunchKernelGGL((matvec_q8_0_once_kernel<EPI, DOT>), dim3((unsigned)groups), dim3(64 * (nw + nq)),
+                       bytes(nw, rw), stream, a.w, a.w2, a.rows, nb, DOT == kInt8 ? a.xs : nullptr,
+                       (const int *)a.xq, a.x, a.arg, nw, nq, rw, a.out);
+    G4_HIP(hipGetLastError());
+    *done = true;
     return G4_OK;
 }
 
@@ -544,20 +744,21 @@ int launch_q8(g4_ctx *ctx, MatvecArgs a, hipStream_t stream) {
     const int num_cus = ctx->num_cus;
     const int64_t nb = a.cols / kQ8Values;
     // Rows start 16-byte aligned when cols is a multiple of 256 and the
-    // matrices are (GGUF aligns tensor data to 32 bytes).
-    const bool aligned = ((uintptr_t)a.w % 16 == 0) && (NM == 1 || (uintptr_t)a.w2 % 16 == 0) &&
-                         (a.xs || (uintptr_t)a.x % 16 == 0);
-    // An empty row (cols == 0) takes the row-wise kernel, which reads no
-    // block: the staged kernel loads the activation's blocks before it tests
-    // them against the block count.
-    const bool fast = a.cols % 256 == 0 && nb > 0 && nb <= 256 && aligned;
+    // matrices are (GGUF aligns tensor data to 32 bytes).  An empty row
+    // (cols == 0) takes the row-wise kernel, which reads no block.
+    const bool aligned = (uintptr_t)a.w % 16 == 0 && (NM == 1 || (uintptr_t)a.w2 % 16 == 0);
+    const bool staged = a.cols % 256 == 0 && nb > 0 && nb <= 256 && aligned;
     // Rows per workgroup: up to 16, the product table under 16 KB.
     const int64_t rb_max = std::min<int64_t>(16, std::max<int64_t>(1, 16384 / (NM * (nb + 1) * 4)));
-    const bool large = a.rows >= rb_max * 8 * num_cus;
-    if (!a.xs && (!fast || large)) {
-        // An f32 activation for a kernel that reads a quantized one, or a
-        // matrix large enough that its many workgroups would each quantize
-        // it again: quantize_q8_0 into the context's workspace first.
+    const bool large = staged && a.rows >= rb_max * 8 * num_cus;
+    if (!large) {
+        bool done = false;
+        const int rc = launch_q8_once<EPI, kInt8>(ctx, a, stream, &done);
+        if (rc != G4_OK || done) return rc;
+    }
+    if (!a.xs) {
+        // An f32 activation for a kernel that reads a quantized one:
+        // quantize_q8_0 into the context's workspace first.
         const size_t sbytes = ((size_t)nb * sizeof(float) + 255) / 256 * 256;
         const int rc = ensure_workspace(ctx, sbytes + (size_t)a.cols, stream);
         if (rc != G4_OK) return rc;
@@ -566,40 +767,34 @@ int launch_q8(g4_ctx *ctx, MatvecArgs a, hipStream_t stream) {
         const int rq = launch_quantize_q8_0(a.x, a.cols, (float *)a.xs, (signed char *)a.xq, stream);
         if (rq != G4_OK) return rq;
     }
-    if (fast) {
-        // Large matrices: 8 rows per workgroup, staged two at a time, so
-        // that the workgroups are small and many are resident per CU, each
-        // with two rows in flight.  Output head (262,144 x 1536, quantize
-        // included): 75.5 us with 16 rows staged one at a time, 71.5 with
-        // 8 (or 4) staged two at a time, 87 with 8 staged eight at a time,
-        // 97-142 with 64 rows per workgroup.  Small ones: a workgroup's rows
-        // all in flight at once, and about eight workgroups per CU.
-        int64_t rb, g;
-        if (large) {
-            rb = std::min<int64_t>(8, rb_max);
-            g = std::min<int64_t>(2, rb);
-        } else {
-            rb = std::max<int64_t>(1, std::min<int64_t>(rb_max, a.rows / (8LL * num_cus)));
-            g = rb;
-        }
-        const int ns = (int)((nb + 63) / 64);
-        if (large) {
-            switch (ns) {
-            case 1: return launch_q8_rows<EPI, 1, true>(a, (int)g, (int)rb, stream);
-            case 2: return launch_q8_rows<EPI, 2, true>(a, (int)g, (int)rb, stream);
-            case 3: return launch_q8_rows<EPI, 3, true>(a, (int)g, (int)rb, stream);
-            default: return launch_q8_rows<EPI, 4, true>(a, (int)g, (int)rb, stream);
-            }
-        }
-        switch (ns) {
-        case 1: return launch_q8_rows<EPI, 1, false>(a, (int)g, (int)rb, stream);
-        case 2: return launch_q8_rows<EPI, 2, false>(a, (int)g, (int)rb, stream);
-        case 3: return launch_q8_rows<EPI, 3, false>(a, (int)g, (int)rb, stream);
-        default: return launch_q8_rows<EPI, 4, false>(a, (int)g, (int)rb, stream);
+    if (large) {
+        // 8 rows per workgroup, staged two at a time, so that the workgroups
+        // are small and many are resident per CU, each with two rows in
+        // flight.  Output head (262,144 x 1536, quantize included): 75.5 us
+        // with 16 rows staged one at a time, 71.5 with 8 (or 4) staged two at
+        // a time, 87 with 8 staged eight at a time, 97-142 with 64 rows per
+        // workgroup.
+        const int rb = (int)std::min<int64_t>(8, rb_max), g = std::min(2, rb);
+        switch ((nb + 63) / 64) {
+        case 1: return launch_q8_rows<EPI, 1>(a, g, rb, stream);
+        case 2: return launch_q8_rows<EPI, 2>(a, g, rb, stream);
+        case 3: return launch_q8_rows<EPI, 3>(a, g, rb, stream);
+        default: return launch_q8_rows<EPI, 4>(a, g, rb, stream);
         }
     }
     hipLaunchKernelGGL((matvec_q8_0_rowwise_kernel<EPI>), dim3((unsigned)((a.rows + 255) / 256)), dim3(256), 0,
                        stream, a.w, a.w2, a.rows, (int)nb, a.xs, (const int *)a.xq, a.arg, a.out);
+    G4_HIP(hipGetLastError());
+    return G4_OK;
+}
+
+template <int DOT>
+int launch_q8_f32(g4_ctx *ctx, const MatvecArgs &a, hipStream_t stream) {
+    bool done = false;
+    const int rc = launch_q8_once<kPlain, DOT>(ctx, a, stream, &done);
+    if (rc != G4_OK || done) return rc;
+    hipLaunchKernelGGL(matvec_q8_0_f32_kernel<DOT == kF64>, dim3((unsigned)((a.rows + 255) / 256)), dim3(256), 0,
+                       stream, a.w, a.rows, (int)(a.cols / kQ8Values), a.x, a.out);
     G4_HIP(hipGetLastError());
     return G4_OK;
 }
@@ -637,24 +832,16 @@ int launch_quantize_q8_0(const float *x, int64_t n, float *scales, signed char *
 
 int launch_matvec(g4_ctx *ctx, const MatvecArgs &a, hipStream_t stream) {
     if (a.rows <= 0) return G4_OK;
-    const unsigned grid = (unsigned)((a.rows + 255) / 256);
     switch (a.kind) {
     case MatvecKind::Q8: return launch_q8<kPlain>(ctx, a, stream);
     case MatvecKind::Q8Softcap: return launch_q8<kSoftcap>(ctx, a, stream);
     case MatvecKind::Q8Geglu: return launch_q8<kGeglu>(ctx, a, stream);
     case MatvecKind::Q8GegluFp16: return launch_q8<kGegluFp16>(ctx, a, stream);
-    case MatvecKind::Q8F32:
-        hipLaunchKernelGGL(matvec_q8_0_f32_kernel<false>, dim3(grid), dim3(256), 0, stream, a.w, a.rows,
-                           (int)(a.cols / kQ8Values), a.x, a.out);
-        break;
-    case MatvecKind::Q8F64:
-        hipLaunchKernelGGL(matvec_q8_0_f32_kernel<true>, dim3(grid), dim3(256), 0, stream, a.w, a.rows,
-                           (int)(a.cols / kQ8Values), a.x, a.out);
-        break;
+    case MatvecKind::Q8F32: return launch_q8_f32<kF32>(ctx, a, stream);
+    case MatvecKind::Q8F64: return launch_q8_f32<kF64>(ctx, a, stream);
     case MatvecKind::Bf16: return launch_dense<unsigned short>(ctx, a, stream);
     case MatvecKind::F32: return launch_dense<float>(ctx, a, stream);
     }
-    G4_HIP(hipGetLastError());
     return G4_OK;
 }
 

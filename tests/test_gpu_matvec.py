@@ -222,6 +222,47 @@ def test_fused_quantization_entries_equal_the_two_step_calls(ctx, rows, cols):
             assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("rows,cols", [(1, 32), (2, 64), (255, 96), (257, 1568), (2047, 160), (2049, 224), (4097, 544),
+                                       (9, 30016), (33000, 64)])
+@pytest.mark.parametrize("shift", [0, 2, 4])
+def test_q8_0_matvecs_at_the_tiles_edges(ctx, rows, cols, shift):
+    """Row counts around the wavefronts' shares, column counts whose rows
+    start anywhere (34-byte blocks, odd block counts), rows too long for one
+    workgroup per CU, and matrices 2 and 4 bytes off a 16-byte boundary: the
+    quantized, the fused and both f32-activation forms, bit for bit."""
+    print(f"[case] q8_0 {rows}x{cols} shift {shift}", flush=True)
+    w = I.q8_0_bytes(np.random.default_rng(rows + cols).uniform(-1.0, 1.0, rows * cols).astype(np.float32))
+    x = np.random.default_rng(cols).standard_normal(cols).astype(np.float32)
+    x[:32] = 0.0
+    d = dev(np.concatenate([np.zeros(shift, np.uint8), w]))[shift:]
+    dx = dev(x)
+    xs, xq = q8_activation(ctx, x)
+    out = torch.full((rows + 1,), 7.0, device="cuda")
+
+    def check(ref, what):
+        got = host(out)
+        assert got[rows] == 7.0 and np.array_equal(got[:rows].view(np.uint32), ref.view(np.uint32)), what
+
+    ref = orc.matvec_q8_0(w, rows, cols, host(xs), host(xq))
+    ctx.matvec_q8_0(d, rows, cols, xs, xq, out)
+    check(ref, "quantized")
+    ctx.project_q8_0(d, rows, cols, dx, out)
+    check(ref, "quantized inside")
+    for f64 in (False, True):
+        ctx.matvec_q8_0_f32(d, rows, cols, dx, out, f64_sums=f64)
+        check(orc.matvec_q8_0_f32(w, rows, cols, x, f64_sums=f64), f"f32 activation, f64 sums {f64}")
+    ctx.geglu_q8_0(d, d, rows, cols, xs, xq, out)
+    gate = host(out).copy()
+    ctx.gated_ffn_q8_0(d, d, rows, cols, dx, out)
+    assert np.array_equal(gate, host(out))
+    assert I.rel_err(gate[:rows], ref * orc_gelu(ref)) < 1e-5
+
+
+def orc_gelu(v):
+    v = v.astype(np.float64)
+    return 0.5 * v * (1.0 + np.tanh(0.7978846 * v * (1.0 + 0.044715 * v * v)))
+
+
 def test_empty_rows(ctx):
     """cols == 0: every output is the empty sum (the reference's -0.0, through
     the soft-cap or the GELU gate), with no element read -- for the calls that
