@@ -1194,18 +1194,25 @@ int launch_mode(g4_ctx *ctx, const DecodeArgs &a, DecodeK p, hipStream_t stream,
     // MFMA tiles.  One sequence: one workgroup per CU (the occupancy of the
     // split kernel), down to a single tile each -- a workgroup's time is
     // its MFMA and softmax work, so spreading the tiles over every CU wins
-    // over fewer, longer splits.  Ragged batches: about eight per CU, at
-    // least 64 keys, so that sequences of very different lengths still
-    // balance over the CUs.  Contexts of up to two tiles run as one split
-    // (no merge); longer ones split even when short: 64 keys took 6.8 us as
-    // one workgroup, 5.7 us as four one-tile splits and the merge.
+    // over fewer, longer splits.  Ragged batches the same, over the batch's
+    // bound (B sequences of max_kv_len): one tile up to one and a half
+    // workgroups per CU, then the nearest whole number of 32-key pairs, since
+    // a part of a pair takes the time of a pair.  Measured (us, splits of
+    // 16 / 32 / 64 keys): 8 x 512 keys d=256 7.5 / 8.6 / 10.8; 16 x 512 11.3 /
+    // 10.2 / 11.6; 32 x 512 17.5 / 15.3 / 13.3; d=512, 8 of up to 579 keys 9.7
+    // / 11.1 / 15.6; 5 of up to 1868 14.7 / 13.3 / 16.4; 26 of up to 636 19.7
+    // / 20.0 / 18.5.  Queries of a prompt: about eight per CU, at least 64
+    // keys.  Contexts of up to two tiles run as one split (no merge); longer
+    // ones split even when short: 64 keys took 6.8 us as one workgroup,
+    // 5.7 us as four one-tile splits and the merge.
     const int64_t units = (int64_t)a.B * a.n_kv_heads;
     const int64_t max_len = a.max_kv_len > 0 ? a.max_kv_len : 1;
     int64_t chunk = ctx->decode_chunk;
     if (chunk <= 0) {
-        const int64_t target = (MODE == kSingle ? 1LL : 8LL) * ctx->num_cus;
+        const int64_t target = (MODE == kPrefill ? 8LL : 1LL) * ctx->num_cus;
         chunk = (max_len * units + target - 1) / target;
-        const int64_t floor_keys = MODE == kSingle ? 16 : 64;
+        if (MODE == kBatch) chunk = chunk <= 24 ? 16 : (chunk + 16) / 32 * 32;
+        const int64_t floor_keys = MODE == kPrefill ? 64 : 16;
         if (chunk < floor_keys) chunk = floor_keys;
         if (max_len <= 32) chunk = max_len;
     }

@@ -92,3 +92,16 @@ def test_ragged_decode_random_batches(ctx, d, window, lens):
         worst = max(worst, I.rel_err(got[s], orc.attend(q[s], K[rows], V[rows], 8, 1)))
     print(f"[parity] ragged sweep d={d} W={window} B={B}: worst rel err {worst:.2e}")
     assert worst <= TOL
+
+
+@pytest.mark.parametrize("d", [256, 512])
+@pytest.mark.parametrize("B,bound", [(1, 33), (3, 90), (12, 512), (13, 512), (23, 512), (24, 512), (63, 512), (7, 2339)])
+def test_ragged_decode_split_sizes(ctx, d, B, bound):
+    """Batches on each side of the lines between split sizes (16 keys, then
+    whole pairs of 32), with sequences of one key, of the bound, and around
+    the sizes' multiples."""
+    near = [1, 15, 16, 17, 31, 32, 33, 48, 64, 65, bound - 1, bound]
+    lens = np.array([min(bound, near[(B + 5 * s) % len(near)]) for s in range(B)], np.int64)
+    lens[B // 2] = bound
+    print(f"[case] ragged splits d={d} B={B} bound={bound}", flush=True)
+    test_ragged_decode_random_batches(ctx, d, 0, lens.tolist())
