@@ -316,6 +316,18 @@ struct PrefillShape {
     static constexpr int TPS = KSPLIT;               // tiles per step, one per wave group
 };
 
+// Slot of dims 4*c4 .. +3 of output row `row` (16 rows of DH floats per
+// wavefront) in the LDS transpose.  A lane holds four consecutive dims, so it
+// writes 16 bytes at a time; swizzled by the row, the 16 lanes of a write,
+// one per row, fall on distinct bank groups, as do those of a read.  Single
+// floats in plain row order put them all on one bank: whole calls at d = 512
+// of 9 queries 17.4 -> 14.5 us, 512 queries 36.2 -> 33.6, 2048 133.7 -> 129.1;
+// at d = 256 14.8 -> 13.5, 28.9 -> 28.0, 45.7 -> 44.4 (the merge included).
+template <int DH>
+__device__ inline int out_slot(int row, int c4) {
+    return row * (DH / 4) + (c4 ^ row);
+}
+
 // One unit: the rows of position block u.block against its key tiles
 // [u.t_lo, u.t_hi), leaving the block's output or the unit's partial.
 // SPLIT16: products as split-f16 MFMAs from the planes; such a unit first
@@ -996,25 +1008,23 @@ __device__ __forceinline__ bool prefill_unit(const PrefillK &p, const PrefillUni
         }
         return true;
     }
-    // Single unit: normalise and write row-major through LDS (coalesced).
+    // Single unit: normalise and write row-major through LDS (coalesced),
+    // each wavefront its own rows.
     __syncthreads();  // every wave is done with the tile buffers (no tile load is in flight)
+    if (!result) return true;
     // RWAVES/4 waves' rows per tile array.
     constexpr int WPA = S::RWAVES / 4;
     static_assert(WPA * kRowsPerWave * DH <= TPS * TILE_F4 * 4 && S::RWAVES % 4 == 0, "transpose fits the tile buffers");
-    const int ta = (result ? wave : 0) / WPA;
+    const int ta = wave / WPA;
     f32x4 *tb = ta == 0 ? lds_k0 : ta == 1 ? lds_v0 : ta == 2 ? lds_k1 : lds_v1;
-    float *tr = (float *)tb + (wave % WPA) * (kRowsPerWave * DH);
+    f32x4 *tr = tb + (wave % WPA) * (kRowsPerWave * DH / 4);
     const float inv = 1.0f / lt;
-    if (result) {
 #pragma unroll
-        for (int U = 0; U < NV; ++U)
+    for (int U = 0; U < NV; ++U)
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) tr[c * DH + 64 * U + 4 * (4 * g + r) + i] = o[4 * U + i][r] * inv;
-    }
-    __syncthreads();
-    if (!result) return true;
+        for (int r = 0; r < 4; ++r)
+            tr[out_slot<DH>(c, 16 * U + 4 * g + r)] =
+                f32x4{o[4 * U][r], o[4 * U + 1][r], o[4 * U + 2][r], o[4 * U + 3][r]} * inv;
 #pragma unroll
     for (int e = 0; e < kRowsPerWave * DH / 4 / 64; ++e) {
         const int f = lane + 64 * e;
@@ -1022,7 +1032,7 @@ __device__ __forceinline__ bool prefill_unit(const PrefillK &p, const PrefillUni
         const int64_t rpos = P0 + kPosPerWave * rg + (row >> 3);
         if (rpos > last_pos) continue;
         float *orow = p.out + ((rpos - p.pos0) * p.n_heads + kvh * kGroup + (row & 7)) * D + d0;
-        *(f32x4 *)(orow + 4 * c4) = *(const f32x4 *)(tr + row * DH + 4 * c4);
+        *(f32x4 *)(orow + 4 * c4) = tr[out_slot<DH>(row, c4)];
     }
     return true;
 }
@@ -1077,7 +1087,7 @@ __global__ __launch_bounds__(PrefillShape<D>::THREADS, 1) void prefill_kernel(Pr
 // thread issues exactly its NU loads per element.
 template <int D, int NU>
 __device__ __forceinline__ void merge_units(const PrefillK &p, const PrefillBlockInfo &bi, float (*w)[kRowsPerWave],
-                                            float *Linv, float *tr) {
+                                            float *Linv, f32x4 *tr) {
     using S = PrefillShape<D>;
     constexpr int DH = S::DH;
     constexpr int NT = DH / 16;
@@ -1086,8 +1096,10 @@ __device__ __forceinline__ void merge_units(const PrefillK &p, const PrefillBloc
     const int tid = threadIdx.x;
     // Every load first (one memory round trip): the wave's (m, l) per row and
     // unit, and this thread's partial vectors.
-    constexpr int NE = NT * 64 / 256;  // vectors per thread
-    static_assert(NT * 64 % 256 == 0, "whole vectors per thread");
+    // Thread (U, lane) takes that lane's vectors of the four O^T tiles of
+    // 64-dim group U, which hold four consecutive dims of a row between them.
+    static_assert(NT == 16, "four groups of four tiles, 256 threads");
+    const int lane = tid & 63, U = tid >> 6, g = lane >> 4, c = lane & 15;
     const int ml_row = rg * kRowsPerWave + (tid & (kRowsPerWave - 1));
     float2 ml[NU];
 #pragma unroll
@@ -1096,11 +1108,11 @@ __device__ __forceinline__ void merge_units(const PrefillK &p, const PrefillBloc
     const f32x4 *base = (const f32x4 *)p.part_o +
                         ((int64_t)bi.first_slot * gridDim.y + kvh) * (kWaves * kRowsPerWave * D / 4) +
                         (int64_t)wave * NT * 64;
-    f32x4 v[NE][NU];
+    f32x4 v[4][NU];
 #pragma unroll
-    for (int k = 0; k < NE; ++k)
+    for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int j = 0; j < NU; ++j) v[k][j] = base[j * slot_stride + tid + 256 * k];
+        for (int j = 0; j < NU; ++j) v[i][j] = base[j * slot_stride + (4 * U + i) * 64 + lane];
     __builtin_amdgcn_sched_barrier(0);  // no wait before every load above is issued
     if (tid < kRowsPerWave) {
         float M = -INFINITY;
@@ -1116,19 +1128,17 @@ __device__ __forceinline__ void merge_units(const PrefillK &p, const PrefillBloc
         Linv[tid] = 1.0f / L;
     }
     __syncthreads();
+    f32x4 acc[4];
+    const float inv = Linv[c];
 #pragma unroll
-    for (int k = 0; k < NE; ++k) {
-        const int e = tid + 256 * k;
-        const int lane = e & 63, tile = e >> 6;
-        const int g = lane >> 4, c = lane & 15;
-        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int i = 0; i < 4; ++i) {
+        acc[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int j = 0; j < NU; ++j) acc += w[j][c] * v[k][j];
-        const int U = tile >> 2, i = tile & 3;
-        const float inv = Linv[c];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) tr[c * DH + 64 * U + 4 * (4 * g + r) + i] = acc[r] * inv;
+        for (int j = 0; j < NU; ++j) acc[i] += w[j][c] * v[i][j];
     }
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+        tr[out_slot<DH>(c, 16 * U + 4 * g + r)] = f32x4{acc[0][r], acc[1][r], acc[2][r], acc[3][r]} * inv;
     __syncthreads();
     const int64_t P0 = p.pos0 + (int64_t)kPosPerBlock * blockIdx.x;
     const int64_t last_pos = p.pos0 + p.N - 1;
@@ -1137,7 +1147,7 @@ __device__ __forceinline__ void merge_units(const PrefillK &p, const PrefillBloc
         const int64_t rpos = P0 + kPosPerWave * rg + (row >> 3);
         if (rpos <= last_pos) {
             float *orow = p.out + ((rpos - p.pos0) * p.n_heads + kvh * kGroup + (row & 7)) * D + half * DH;
-            *(f32x4 *)(orow + 4 * c4) = *(const f32x4 *)(tr + row * DH + 4 * c4);
+            *(f32x4 *)(orow + 4 * c4) = tr[out_slot<DH>(row, c4)];
         }
     }
 }
@@ -1146,7 +1156,7 @@ template <int D>
 __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillK p) {
     __shared__ float w[kPrefillMaxUnitsDev][kRowsPerWave];
     __shared__ float Linv[kRowsPerWave];
-    __shared__ float tr[kRowsPerWave * PrefillShape<D>::DH];
+    __shared__ f32x4 tr[kRowsPerWave * PrefillShape<D>::DH / 4];
     const PrefillBlockInfo bi = p.blocks[blockIdx.x];
     static_assert(kPrefillMaxUnitsDev == 8, "one case per unit count");
     switch (bi.n_units) {  // uniform; 0 or 1 unit: nothing to merge
