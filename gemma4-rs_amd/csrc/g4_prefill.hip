@@ -33,6 +33,7 @@
 #include <algorithm>
 #include <cmath>
 #include <array>
+#include <climits>
 #include <functional>
 #include <queue>
 #include <utility>
@@ -139,6 +140,7 @@ struct PrefillK {
     float *part_o;    // [slot][kv head][wave][D/16 tiles][64 lanes] f32x4
     float2 *part_ml;  // [slot][kv head][64 rows]
     int n_slots;
+    int slices;  // workgroups (blockIdx.z) that share each unit's tiles
     unsigned *status;
     // Split-f16 planes of K and V (null: every unit uses f32 MFMAs):
     // [tile - t0][kv head][K block | V block], each block 16 keys x D dims
@@ -1072,7 +1074,13 @@ __global__ __launch_bounds__(PrefillShape<D>::THREADS, 1) void prefill_kernel(Pr
         // The previous unit's waves are done with the tile buffers (its
         // spare tile loads landed before its epilogue).
         if (i > first) __syncthreads();
-        const PrefillUnit u = p.units[i];
+        PrefillUnit u = p.units[i];
+        if (p.slices > 1) {  // this workgroup's share (the host leaves each at least one tile)
+            const int n = u.t_hi - u.t_lo, z = blockIdx.z, lo = u.t_lo;
+            u.t_lo = lo + n * z / p.slices;
+            u.t_hi = lo + n * (z + 1) / p.slices;
+            u.slot = u.slot * p.slices + z;
+        }
         if (p.planes != nullptr && prefill_unit<D, true>(p, u, L)) continue;
         if (p.planes != nullptr) __syncthreads();  // the declined split form's tiles have landed
         prefill_unit<D, false>(p, u, L);
@@ -1171,13 +1179,87 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillK p) {
     }
 }
 
+// The merge of blocks cut into more pieces than merge_units takes (units
+// times slices): a workgroup takes one wavefront's rows and one 64-dim group
+// (blockIdx.z: wavefront, group), and its four wavefronts fold every fourth
+// piece, kMergeBatch loads of pieces in flight, before they are combined in
+// a fixed order.  (One workgroup for all of a wavefront's dims would read
+// up to 4 MB through one CU.)
+constexpr int kMergeBatch = 4;
+
+template <int D>
+__global__ __launch_bounds__(256) void prefill_merge_many_kernel(PrefillK p) {
+    using S = PrefillShape<D>;
+    constexpr int DH = S::DH, NT = DH / 16, NG = NT / 4;
+    const PrefillBlockInfo bi = p.blocks[blockIdx.x];
+    const int n = bi.n_units, kvh = blockIdx.y, wave = blockIdx.z / NG, U = blockIdx.z % NG;
+    const int rg = wave % kWaves, half = wave / kWaves;
+    const int ph = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
+    const int64_t slot0 = (int64_t)bi.first_slot * gridDim.y + kvh;
+    const int64_t slot_stride = (int64_t)gridDim.y * kWaves * kRowsPerWave * D / 4;  // f32x4
+    const f32x4 *base = (const f32x4 *)p.part_o + slot0 * (kWaves * kRowsPerWave * D / 4) +
+                        (int64_t)(wave * NT + 4 * U) * 64 + lane;
+    const float2 *mls = p.part_ml + slot0 * 64 + rg * kRowsPerWave + c;
+    float m = -INFINITY, l = 0.0f;
+    f32x4 o[4] = {};
+    // (m, l, o) and (m2, l2, o2) over disjoint keys, into the first.
+    auto fold = [&](float m2, float l2, const f32x4 (&o2)[4]) {
+        const float mm = fmaxf(m, m2);
+        const float a = m == -INFINITY ? 0.0f : exp2_fast((m - mm) * kLog2e);
+        const float b = m2 == -INFINITY ? 0.0f : exp2_fast((m2 - mm) * kLog2e);
+        l = a * l + b * l2;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[i] = a * o[i] + b * o2[i];
+        m = mm;
+    };
+    for (int j0 = ph; j0 < n; j0 += 4 * kMergeBatch) {
+        float2 ml[kMergeBatch];
+        f32x4 v[kMergeBatch][4];
+#pragma unroll
+        for (int b = 0; b < kMergeBatch; ++b) {
+            const int j = min(j0 + 4 * b, n - 1);
+            ml[b] = mls[(int64_t)j * gridDim.y * 64];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[b][i] = base[j * slot_stride + 64 * i];
+        }
+        __builtin_amdgcn_sched_barrier(0);  // no wait before every load above is issued
+#pragma unroll
+        for (int b = 0; b < kMergeBatch; ++b)
+            if (j0 + 4 * b < n) fold(ml[b].x, ml[b].y, v[b]);
+    }
+    __shared__ f32x4 red[3][4][64];
+    __shared__ float2 red_ml[3][64];
+    if (ph > 0) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) red[ph - 1][i][lane] = o[i];
+        red_ml[ph - 1][lane] = float2{m, l};
+    }
+    __syncthreads();
+    if (ph > 0) return;
+    for (int w = 0; w < 3; ++w) {
+        f32x4 o2[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o2[i] = red[w][i][lane];
+        fold(red_ml[w][lane].x, red_ml[w][lane].y, o2);
+    }
+    const int64_t rpos = p.pos0 + (int64_t)kPosPerBlock * blockIdx.x + kPosPerWave * rg + (c >> 3);
+    if (rpos >= p.pos0 + p.N) return;
+    float *orow = p.out + ((rpos - p.pos0) * p.n_heads + kvh * kGroup + (c & 7)) * D + half * DH + 64 * U + 16 * g;
+    const float inv = 1.0f / l;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) *(f32x4 *)(orow + 4 * r) = f32x4{o[0][r], o[1][r], o[2][r], o[3][r]} * inv;
+}
+
 constexpr int kPrefillMaxUnits = kPrefillMaxUnitsDev;  // per position block
 
 // A unit table in device memory, for one prefill shape.
 struct PrefillPlan {
     int64_t pos0 = -1, N = -1, window = -1;
     int head_dim = 0, n_kv_heads = 0;
+    bool split = false;
     int n_units = 0, n_bins = 0, n_blocks = 0, n_slots = 0;
+    int slices = 1;     // workgroups per unit
+    int max_parts = 1;  // partials of a block, at most
     PrefillUnit *units = nullptr;
     int *bin_start = nullptr;
     PrefillBlockInfo *blocks = nullptr;
@@ -1228,47 +1310,76 @@ void release_prefill_plan(g4_ctx *ctx) {
 // key ranges is chosen knowing where each piece runs.
 //
 // Cost model, in tiles (one 16-key tile of 64 query rows): a unit costs its
-// tiles plus kUnitCost (loading Q, filling the tile pipeline, writing O or
-// the partial); blocks split into several units add a merge kernel of
-// kMergeBase + kMergePerPartial per partial.  Measured on MI355X at
-// d = 512: 4.9 us per tile, 9.1 us per unit (the fit over a 2048-token
-// causal prompt's 480 units), merge 17 us for 384 partials.
-constexpr double kUnitCost = 1.9;
-constexpr double kMergePerPartial = 0.009;
+// tiles plus `unit` (loading Q, filling the tile pipeline, writing O or the
+// partial); blocks split into several units add a merge kernel of
+// merge_base + merge_per_partial per partial.  f32 form, measured on MI355X
+// at d = 512: 4.9 us per tile, 9.1 us per unit (the fit over a 2048-token
+// causal prompt's 480 units), merge 17 us for 384 partials.  The split form's
+// tiles take 1.9 us (0.85 at d = 256, two per step) and its units about 9 us
+// still, so they weigh more; its constants are the lowest of sweeps over
+// unit 1.9 .. 14 and merge base 0.6 .. 8 (whole calls, f32 constants ->
+// these, us): d = 256, 1024 queries 48.2 -> 35.9, 1500 56.2 -> 41.8; d = 512,
+// 777 queries 48.0 -> 44.7, 1024 61.4 -> 55.9, 1500 96.1 -> 89.7.
+struct ScheduleCost {
+    double unit, merge_base, merge_per_partial;
+};
+static ScheduleCost cost_of(int head_dim, bool split) {
+    if (split) return head_dim == 512 ? ScheduleCost{7.0, 1.0, 0.012} : ScheduleCost{12.0, 3.0, 0.02};
+    return ScheduleCost{1.9, head_dim == 512 ? 0.6 : 1.2, 0.009};
+}
 constexpr int kMinUnitTiles = 4;  // a split leaves no piece shorter (unless the block is)
+// A block has at most kPrefillMaxUnits units; where those do not fill the
+// chip (few positions deep in a context), each unit's tiles are shared out
+// once more, over `slices` workgroups.  More pieces per block than the merge
+// kernel's registers hold cost it another pass per 16.
+constexpr double kMergePass = 0.5;
 
 using Piece = std::array<int, 3>;  // block, t_lo, t_hi
 using Bins = std::vector<std::vector<Piece>>;
 
-static double merge_cost(int partials, int head_dim) {
-    if (partials == 0) return 0.0;
-    return (head_dim == 512 ? 0.6 : 1.2) + kMergePerPartial * partials;
-}
-
-// Makespan plus merge cost; nullopt-like -1 when a block has more pieces
-// than the merge kernel combines.
-static double schedule_cost(const Bins &bins, int n_blocks, int head_dim) {
+// Makespan plus merge cost with the best number of slices for up to n_bins
+// workgroups per KV head; -1 when a block has more pieces than allowed.
+static double schedule_cost(const Bins &bins, int n_blocks, int n_bins, const ScheduleCost &sc, int *slices) {
     std::vector<int> pieces(n_blocks, 0);
-    double makespan = 0.0;
+    int used = 0, min_tiles = INT_MAX, units = 0;
     for (auto &bin : bins) {
-        double load = 0.0;
+        used += !bin.empty();
         for (auto &pc : bin) {
-            load += pc[2] - pc[1] + kUnitCost;
+            min_tiles = std::min(min_tiles, pc[2] - pc[1]);
             ++pieces[pc[0]];
+            ++units;
         }
-        makespan = std::max(makespan, load);
     }
-    int partials = 0;
+    int partials = 0, most = 0;
     for (int n : pieces) {
         if (n > kPrefillMaxUnits) return -1.0;
         if (n > 1) partials += n;
+        most = std::max(most, n);
     }
-    return makespan + merge_cost(partials, head_dim);
+    double best = -1.0;
+    const int top = std::max(1, std::min(used > 0 ? n_bins / used : 1, min_tiles / kMinUnitTiles));
+    for (int s = 1; s <= top; ++s) {
+        double makespan = 0.0;
+        for (auto &bin : bins) {
+            double load = 0.0;
+            for (auto &pc : bin) load += (pc[2] - pc[1] + s - 1) / s + sc.unit;
+            makespan = std::max(makespan, load);
+        }
+        const int parts = s == 1 ? partials : units * s;
+        const double merge = parts == 0 ? 0.0
+                                        : sc.merge_base + sc.merge_per_partial * parts +
+                                              (most * s > kPrefillMaxUnits ? kMergePass * ((most * s + 15) / 16) : 0.0);
+        if (best < 0.0 || makespan + merge < best) {
+            best = makespan + merge;
+            *slices = s;
+        }
+    }
+    return best;
 }
 
 // Fixed-length units (each block cut into ceil(tiles / ut) near-equal
 // pieces) assigned heaviest first to the least loaded bin.
-static Bins lpt_bins(const std::vector<std::pair<int, int>> &bt, int ut, int n_bins) {
+static Bins lpt_bins(const std::vector<std::pair<int, int>> &bt, int ut, int n_bins, const ScheduleCost &sc) {
     std::vector<Piece> units;
     for (int b = 0; b < (int)bt.size(); ++b) {
         const int t_lo = bt[b].first, tiles = bt[b].second - t_lo, nu = (tiles + ut - 1) / ut;
@@ -1284,7 +1395,7 @@ static Bins lpt_bins(const std::vector<std::pair<int, int>> &bt, int ut, int n_b
         Load l = heap.top();
         heap.pop();
         bins[l.second].push_back(u);
-        heap.push({l.first + (u[2] - u[1]) + kUnitCost, l.second});
+        heap.push({l.first + (u[2] - u[1]) + sc.unit, l.second});
     }
     return bins;
 }
@@ -1293,7 +1404,8 @@ static Bins lpt_bins(const std::vector<std::pair<int, int>> &bt, int ut, int n_b
 // smallest, second largest, second smallest, ... fill the bins in turn; a
 // block that does not fit is cut at the capacity and continues in the next
 // bin.  False when more than n_bins bins are needed.
-static bool stream_bins(const std::vector<std::pair<int, int>> &bt, double cap, int n_bins, Bins &bins) {
+static bool stream_bins(const std::vector<std::pair<int, int>> &bt, double cap, int n_bins, const ScheduleCost &sc,
+                        Bins &bins) {
     std::vector<int> order(bt.size());
     for (size_t i = 0; i < order.size(); ++i) order[i] = (int)i;
     std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
@@ -1311,12 +1423,12 @@ static bool stream_bins(const std::vector<std::pair<int, int>> &bt, double cap, 
         const int hi = bt[b].second;
         while (lo < hi) {
             const int rem = hi - lo;
-            const double room = cap - load - kUnitCost;
+            const double room = cap - load - sc.unit;
             const bool empty = bins.back().empty();
             // An empty bin takes any remainder up to a minimum piece whole.
             if (rem <= room || (empty && rem <= kMinUnitTiles)) {
                 bins.back().push_back({b, lo, hi});
-                load += rem + kUnitCost;
+                load += rem + sc.unit;
                 break;
             }
             // The tiles that fit, leaving at least a minimum piece behind
@@ -1345,7 +1457,8 @@ static bool stream_bins(const std::vector<std::pair<int, int>> &bt, double cap, 
 // feasible capacity or a little above.  Stream-K wins on causal prompts
 // (every CU gets the same number of tiles, with about one split per CU);
 // LPT wins where few long blocks each need many pieces.
-static int build_schedule(const std::vector<std::pair<int, int>> &bt, int n_bins, int head_dim, Bins &best) {
+static int build_schedule(const std::vector<std::pair<int, int>> &bt, int n_bins, const ScheduleCost &sc, Bins &best,
+                          int *slices) {
     int max_tiles = 1;
     long long total = 0;
     for (auto &x : bt) {
@@ -1354,29 +1467,31 @@ static int build_schedule(const std::vector<std::pair<int, int>> &bt, int n_bins
     }
     double best_cost = -1.0;
     auto consider = [&](Bins &&bins) {
-        const double cost = schedule_cost(bins, (int)bt.size(), head_dim);
+        int s = 1;
+        const double cost = schedule_cost(bins, (int)bt.size(), n_bins, sc, &s);
         if (cost >= 0.0 && (best_cost < 0.0 || cost < best_cost)) {
             best_cost = cost;
             best = std::move(bins);
+            *slices = s;
         }
     };
     const int ut_hi = std::max(128, ((max_tiles + kPrefillMaxUnits - 1) / kPrefillMaxUnits + 7) / 8 * 8);
     for (int ut = ut_hi; ut >= 16; ut -= 8) {
         if ((max_tiles + ut - 1) / ut > kPrefillMaxUnits) break;
-        consider(lpt_bins(bt, ut, n_bins));
+        consider(lpt_bins(bt, ut, n_bins, sc));
     }
-    double lo = (double)total / n_bins + kUnitCost, hi = lo + max_tiles + 2 * kUnitCost;
+    double lo = (double)total / n_bins + sc.unit, hi = lo + max_tiles + 2 * sc.unit;
     Bins bins;
-    if (stream_bins(bt, hi, n_bins, bins)) {
+    if (stream_bins(bt, hi, n_bins, sc, bins)) {
         while (hi - lo > 0.25) {
             const double mid = 0.5 * (lo + hi);
-            if (stream_bins(bt, mid, n_bins, bins))
+            if (stream_bins(bt, mid, n_bins, sc, bins))
                 hi = mid;
             else
                 lo = mid;
         }
         for (int k = 0; k < 12; ++k)
-            if (stream_bins(bt, hi + 0.5 * k, n_bins, bins)) consider(std::move(bins));
+            if (stream_bins(bt, hi + 0.5 * k, n_bins, sc, bins)) consider(std::move(bins));
     }
     return best_cost < 0.0 ? -1 : 0;
 }
@@ -1442,19 +1557,20 @@ static int bins_for(int num_cus, int n_kv_heads) { return std::max(1, num_cus / 
 
 // The schedule tables of a's shape: cached, or built and uploaded
 // (synchronously: graph capture needs an earlier call with the same shape).
-static int plan_for(g4_ctx *ctx, const PrefillArgs &a, const PrefillPlan **out) {
+static int plan_for(g4_ctx *ctx, const PrefillArgs &a, bool split, const PrefillPlan **out) {
     PrefillPlans &ps = plans_of(ctx);
     ++ps.tick;
     for (auto &pl : ps.plans)
         if (pl.pos0 == a.pos0 && pl.N == a.N && pl.window == a.window && pl.head_dim == a.head_dim &&
-            pl.n_kv_heads == a.n_kv_heads) {
+            pl.n_kv_heads == a.n_kv_heads && pl.split == split) {
             pl.last_use = ps.tick;
             *out = &pl;
             return G4_OK;
         }
     const std::vector<std::pair<int, int>> bt = block_tile_ranges(a.pos0, a.N, a.window);
     Bins bins;
-    if (build_schedule(bt, bins_for(ctx->num_cus, a.n_kv_heads), a.head_dim, bins) != 0)
+    int slices = 1;
+    if (build_schedule(bt, bins_for(ctx->num_cus, a.n_kv_heads), cost_of(a.head_dim, split), bins, &slices) != 0)
         return set_error(G4_ERR_COMPUTE, "prefill key range too long for one call");
     std::vector<PrefillUnit> units;
     std::vector<int> bin_start;
@@ -1463,6 +1579,18 @@ static int plan_for(g4_ctx *ctx, const PrefillArgs &a, const PrefillPlan **out) 
     int rc = schedule_tables(bt, bins, units, bin_start, blocks, n_slots);
     if (rc != G4_OK) return rc;
     PrefillPlan pl;
+    if (slices > 1) {  // every unit leaves a partial per slice
+        for (PrefillUnit &u : units)
+            if (u.slot < 0) {
+                u.slot = n_slots++;
+                blocks[u.block] = {u.slot, 1};
+            }
+        for (PrefillBlockInfo &b : blocks) b = {b.first_slot * slices, b.n_units * slices};
+        n_slots *= slices;
+    }
+    for (const PrefillBlockInfo &b : blocks) pl.max_parts = std::max(pl.max_parts, b.n_units);
+    pl.slices = slices;
+    pl.split = split;
     pl.pos0 = a.pos0;
     pl.N = a.N;
     pl.window = a.window;
@@ -1507,7 +1635,8 @@ int describe_prefill_schedule(int64_t pos0, int64_t N, int64_t window, int head_
                               int32_t *counts) {
     const std::vector<std::pair<int, int>> bt = block_tile_ranges(pos0, N, window);
     Bins bins;
-    if (build_schedule(bt, bins_for(num_cus, n_kv_heads), head_dim, bins) != 0)
+    int slices = 1;
+    if (build_schedule(bt, bins_for(num_cus, n_kv_heads), cost_of(head_dim, true), bins, &slices) != 0)
         return set_error(G4_ERR_COMPUTE, "prefill key range too long for one call");
     std::vector<PrefillUnit> units;
     std::vector<int> bin_start;
@@ -1556,8 +1685,19 @@ int launch_prefill(g4_ctx *ctx, const PrefillArgs &a, hipStream_t stream) {
         d.out = a.out;
         return launch_decode(ctx, d, stream);
     }
+    const int D = a.head_dim;
+    const int64_t row_lo = (a.window > 0 && a.pos0 + 1 > a.window) ? a.pos0 + 1 - a.window : 0;
+    const int64_t row_hi = a.pos0 + a.N;
+    const int64_t t0 = row_lo / 16, n_tiles = (row_hi - 1) / 16 + 1 - t0;
+    const size_t plane_bytes = (size_t)n_tiles * a.n_kv_heads * 128 * D;
+    // The split form: f16 products carry any |x| < 2^15 to f32 accuracy; the
+    // planes are addressed with 32-bit offsets; a scale beyond 2^32 could
+    // take scores near the f32 limit, where only the f32 form's rounding is
+    // the reference's.
+    const bool split = !ctx->prefill_exact && plane_bytes < (1ull << 31) && std::isfinite(a.scale) &&
+                       std::fabs(a.scale) <= 4294967296.0f;
     const PrefillPlan *plp = nullptr;
-    int rc = plan_for(ctx, a, &plp);
+    int rc = plan_for(ctx, a, split, &plp);
     if (rc != G4_OK) return rc;
     const PrefillPlan &pl = *plp;
     PrefillK p{};
@@ -1576,24 +1716,14 @@ int launch_prefill(g4_ctx *ctx, const PrefillArgs &a, hipStream_t stream) {
     p.bin_start = pl.bin_start;
     p.blocks = pl.blocks;
     p.n_slots = pl.n_slots;
+    p.slices = pl.slices;
     p.status = ctx->status_dev;
-    const int D = a.head_dim;
     // Workspace: the partials of split blocks, then the split-f16 planes of
     // the attended rows and their tile flags.
     auto up = [](size_t x) { return (x + 255) / 256 * 256; };
     const size_t per_slot = (size_t)a.n_kv_heads * kWaves * kRowsPerWave;
     const size_t obytes = up((size_t)pl.n_slots * per_slot * D * sizeof(float));
     const size_t mlbytes = up((size_t)pl.n_slots * per_slot * sizeof(float2));
-    const int64_t row_lo = (a.window > 0 && a.pos0 + 1 > a.window) ? a.pos0 + 1 - a.window : 0;
-    const int64_t row_hi = a.pos0 + a.N;
-    const int64_t t0 = row_lo / 16, n_tiles = (row_hi - 1) / 16 + 1 - t0;
-    const size_t plane_bytes = (size_t)n_tiles * a.n_kv_heads * 128 * D;
-    // The split form: f16 products carry any |x| < 2^15 to f32 accuracy; the
-    // planes are addressed with 32-bit offsets; a scale beyond 2^32 could
-    // take scores near the f32 limit, where only the f32 form's rounding is
-    // the reference's.
-    const bool split = !ctx->prefill_exact && plane_bytes < (1ull << 31) && std::isfinite(a.scale) &&
-                       std::fabs(a.scale) <= 4294967296.0f;
     const size_t bytes = obytes + mlbytes + (split ? up(plane_bytes) + up((size_t)n_tiles * a.n_kv_heads * 8) : 0);
     if (bytes > 0) {
         rc = ensure_workspace(ctx, bytes, stream);
@@ -1626,13 +1756,23 @@ int launch_prefill(g4_ctx *ctx, const PrefillArgs &a, hipStream_t stream) {
             hipLaunchKernelGGL(prefill_split_kernel<512>, sg, dim3(256), 0, stream, s);
         G4_HIP(hipGetLastError());
     }
-    dim3 grid((unsigned)pl.n_bins, (unsigned)a.n_kv_heads);
+    dim3 grid((unsigned)pl.n_bins, (unsigned)a.n_kv_heads, (unsigned)pl.slices);
     if (D == 256)
         hipLaunchKernelGGL(prefill_kernel<256>, grid, dim3(PrefillShape<256>::THREADS), 0, stream, p);
     else
         hipLaunchKernelGGL(prefill_kernel<512>, grid, dim3(PrefillShape<512>::THREADS), 0, stream, p);
     G4_HIP(hipGetLastError());
-    if (pl.n_slots > 0) {
+    if (pl.max_parts > kPrefillMaxUnits) {
+        // Per producing wavefront of a block and 64-dim group.
+        constexpr int z256 = PrefillShape<256>::RWAVES * PrefillShape<256>::DH / 64;
+        constexpr int z512 = PrefillShape<512>::RWAVES * PrefillShape<512>::DH / 64;
+        const dim3 mgrid((unsigned)pl.n_blocks, (unsigned)a.n_kv_heads, D == 256 ? z256 : z512);
+        if (D == 256)
+            hipLaunchKernelGGL(prefill_merge_many_kernel<256>, mgrid, dim3(256), 0, stream, p);
+        else
+            hipLaunchKernelGGL(prefill_merge_many_kernel<512>, mgrid, dim3(256), 0, stream, p);
+        G4_HIP(hipGetLastError());
+    } else if (pl.n_slots > 0) {
         // One merge workgroup per producing wavefront of a block.
         if (D == 256)
             hipLaunchKernelGGL(prefill_merge_kernel<256>,

@@ -119,3 +119,22 @@ def test_large_scores(ctx, d, window, scale):
         print(f"[parity] x{scale} {form}: vs oracle {w_ref:.2e}, vs f64 {w_64:.2e}; oracle vs f64 {floor:.2e}",
               flush=True)
         assert w_ref <= TOL or w_64 <= 2.0 * floor, form
+
+
+@pytest.mark.parametrize("d,window,pos0,N,exact", [(512, 0, 16384, 8, 0), (512, 0, 4000, 64, 0), (512, 0, 2500, 17, 0),
+                                                   (512, 0, 300, 1, 0), (256, 0, 9000, 9, 0), (256, 512, 5000, 25, 0),
+                                                   (512, 0, 6001, 30, 1), (256, 4096, 7000, 40, 0)])
+def test_few_queries_deep_in_a_context(ctx, d, window, pos0, N, exact):
+    """Few position blocks over many keys: the blocks' units are shared out
+    again over slices, up to one workgroup per CU, and merged from more
+    pieces than the usual merge takes.  Every row against the oracle; rows
+    before the window hold NaN."""
+    print(f"[case] few queries d={d} W={window} pos0={pos0} N={N} exact={exact}", flush=True)
+    q, K, V = case(pos0 + N, pos0 + N, d, pos0)
+    lo = max(0, pos0 + 1 - window) if window else 0
+    gk, gv = K.copy(), V.copy()
+    gk[:lo], gv[:lo] = np.nan, np.nan
+    got = run(ctx, q, gk, gv, pos0, N, window, d, exact)
+    ref, status = orc.attend_prefill(q, K, V, pos0, window, 8, 1)
+    assert not status.any()
+    assert max(I.rel_err(got[i], ref[i]) for i in range(N)) <= TOL
