@@ -34,6 +34,7 @@
 #include <cmath>
 #include <array>
 #include <climits>
+#include <cstring>
 #include <functional>
 #include <queue>
 #include <utility>
@@ -1260,30 +1261,26 @@ struct PrefillPlan {
     int n_units = 0, n_bins = 0, n_blocks = 0, n_slots = 0;
     int slices = 1;     // workgroups per unit
     int max_parts = 1;  // partials of a block, at most
+    void *mem = nullptr;  // the three tables below, one allocation
+    size_t mem_bytes = 0;
     PrefillUnit *units = nullptr;
-    int *bin_start = nullptr;
     PrefillBlockInfo *blocks = nullptr;
+    int *bin_start = nullptr;
     uint64_t last_use = 0;
 };
 
-// The context's tables for the last few shapes (a layer-by-layer prompt
-// alternates sliding and global shapes).  A cached table is never written
-// again, so kernels still in flight on any stream keep reading a valid
-// table; only evicting one waits for the device.
-constexpr size_t kPrefillPlans = 8;
+// The context's tables for the last shapes.  A layer-by-layer prompt alternates
+// sliding and global shapes, two new ones per chunk, and comes back to them for
+// every prompt of its chunk size: 64 chunks' tables (10 KB or so each) stay.
+// With 8, a 2048-token prompt in chunks of 256 rebuilt every table on every
+// pass (2.2 ms for one layer of each kind).  A cached table is never written
+// again, so kernels still in flight on any stream keep reading a valid table;
+// only evicting one waits for the device.
+constexpr size_t kPrefillPlans = 128;
 struct PrefillPlans {
     std::vector<PrefillPlan> plans;
     uint64_t tick = 0;
 };
-
-void free_plan(PrefillPlan &pl) {
-    if (pl.units) (void)hipFree(pl.units);
-    if (pl.bin_start) (void)hipFree(pl.bin_start);
-    if (pl.blocks) (void)hipFree(pl.blocks);
-    pl.units = nullptr;
-    pl.bin_start = nullptr;
-    pl.blocks = nullptr;
-}
 
 }  // namespace
 
@@ -1297,7 +1294,8 @@ static PrefillPlans &plans_of(g4_ctx *ctx) {
 void release_prefill_plan(g4_ctx *ctx) {
     if (!ctx->prefill_plan) return;
     auto *ps = static_cast<PrefillPlans *>(ctx->prefill_plan);
-    for (auto &pl : ps->plans) free_plan(pl);
+    for (auto &pl : ps->plans)
+        if (pl.mem) (void)hipFree(pl.mem);
     delete ps;
     ctx->prefill_plan = nullptr;
 }
@@ -1335,88 +1333,109 @@ constexpr int kMinUnitTiles = 4;  // a split leaves no piece shorter (unless the
 constexpr double kMergePass = 0.5;
 
 using Piece = std::array<int, 3>;  // block, t_lo, t_hi
+using BlockTiles = std::vector<std::pair<int, int>>;  // [t_lo, t_hi) per block
 using Bins = std::vector<std::vector<Piece>>;
 
-// Makespan plus merge cost with the best number of slices for up to n_bins
-// workgroups per KV head; -1 when a block has more pieces than allowed.
-static double schedule_cost(const Bins &bins, int n_blocks, int n_bins, const ScheduleCost &sc, int *slices) {
-    std::vector<int> pieces(n_blocks, 0);
-    int used = 0, min_tiles = INT_MAX, units = 0;
-    for (auto &bin : bins) {
-        used += !bin.empty();
-        for (auto &pc : bin) {
-            min_tiles = std::min(min_tiles, pc[2] - pc[1]);
-            ++pieces[pc[0]];
-            ++units;
-        }
+// Pieces of blocks and the workgroup (bin) each runs on, in run order.  Flat,
+// so that trying a schedule allocates nothing once the vectors have grown.
+struct Packing {
+    std::vector<Piece> pieces;
+    std::vector<int> bin;
+    int used = 0;  // bins with pieces: 0 .. used - 1
+    int slices = 1;
+    double cost = -1.0;
+    void clear() {
+        pieces.clear();
+        bin.clear();
+        used = 0;
+    }
+    void add(int b, const Piece &p) {
+        pieces.push_back(p);
+        bin.push_back(b);
+        used = std::max(used, b + 1);
+    }
+};
+
+struct ScheduleScratch {
+    std::vector<int> parts;
+    std::vector<double> load;
+};
+
+// Sets the packing's cost -- makespan plus merge, with the best number of
+// slices for up to n_bins workgroups per KV head -- or -1 when a block has
+// more pieces than allowed.
+static void price(Packing &k, int n_blocks, int n_bins, const ScheduleCost &sc, ScheduleScratch &tmp) {
+    k.cost = -1.0;
+    tmp.parts.assign(n_blocks, 0);
+    int min_tiles = INT_MAX;
+    for (const Piece &pc : k.pieces) {
+        min_tiles = std::min(min_tiles, pc[2] - pc[1]);
+        ++tmp.parts[pc[0]];
     }
     int partials = 0, most = 0;
-    for (int n : pieces) {
-        if (n > kPrefillMaxUnits) return -1.0;
+    for (int n : tmp.parts) {
+        if (n > kPrefillMaxUnits) return;
         if (n > 1) partials += n;
         most = std::max(most, n);
     }
-    double best = -1.0;
-    const int top = std::max(1, std::min(used > 0 ? n_bins / used : 1, min_tiles / kMinUnitTiles));
+    const int top = std::max(1, std::min(k.used > 0 ? n_bins / k.used : 1, min_tiles / kMinUnitTiles));
     for (int s = 1; s <= top; ++s) {
-        double makespan = 0.0;
-        for (auto &bin : bins) {
-            double load = 0.0;
-            for (auto &pc : bin) load += (pc[2] - pc[1] + s - 1) / s + sc.unit;
-            makespan = std::max(makespan, load);
-        }
-        const int parts = s == 1 ? partials : units * s;
+        tmp.load.assign(k.used, 0.0);
+        for (size_t i = 0; i < k.pieces.size(); ++i)
+            tmp.load[k.bin[i]] += (k.pieces[i][2] - k.pieces[i][1] + s - 1) / s + sc.unit;
+        const double makespan = *std::max_element(tmp.load.begin(), tmp.load.end());
+        const int parts = s == 1 ? partials : (int)k.pieces.size() * s;
         const double merge = parts == 0 ? 0.0
                                         : sc.merge_base + sc.merge_per_partial * parts +
                                               (most * s > kPrefillMaxUnits ? kMergePass * ((most * s + 15) / 16) : 0.0);
-        if (best < 0.0 || makespan + merge < best) {
-            best = makespan + merge;
-            *slices = s;
+        if (k.cost < 0.0 || makespan + merge < k.cost) {
+            k.cost = makespan + merge;
+            k.slices = s;
         }
     }
-    return best;
 }
 
-// Fixed-length units (each block cut into ceil(tiles / ut) near-equal
+// Units of at most ut tiles (each block cut into ceil(tiles / ut) near-equal
 // pieces) assigned heaviest first to the least loaded bin.
-static Bins lpt_bins(const std::vector<std::pair<int, int>> &bt, int ut, int n_bins, const ScheduleCost &sc) {
-    std::vector<Piece> units;
+static void lpt_pack(const BlockTiles &bt, int ut, int n_bins, const ScheduleCost &sc, Packing &k) {
+    k.clear();
     for (int b = 0; b < (int)bt.size(); ++b) {
         const int t_lo = bt[b].first, tiles = bt[b].second - t_lo, nu = (tiles + ut - 1) / ut;
-        for (int j = 0; j < nu; ++j) units.push_back({b, t_lo + j * tiles / nu, t_lo + (j + 1) * tiles / nu});
+        for (int j = 0; j < nu; ++j) k.pieces.push_back({b, t_lo + j * tiles / nu, t_lo + (j + 1) * tiles / nu});
     }
-    std::stable_sort(units.begin(), units.end(),
+    std::stable_sort(k.pieces.begin(), k.pieces.end(),
                      [](const Piece &x, const Piece &y) { return x[2] - x[1] > y[2] - y[1]; });
-    Bins bins((size_t)n_bins);
+    const int n = (int)k.pieces.size();
+    k.bin.resize(n);
+    k.used = std::min(n, n_bins);
     using Load = std::pair<double, int>;
-    std::priority_queue<Load, std::vector<Load>, std::greater<Load>> heap;
-    for (int i = 0; i < n_bins; ++i) heap.push({0.0, i});
-    for (auto &u : units) {
-        Load l = heap.top();
-        heap.pop();
-        bins[l.second].push_back(u);
-        heap.push({l.first + (u[2] - u[1]) + sc.unit, l.second});
+    std::vector<Load> heap;  // after the first n_bins pieces, one to a bin
+    heap.reserve(n_bins);
+    for (int i = 0; i < n; ++i) {
+        const double cost = k.pieces[i][2] - k.pieces[i][1] + sc.unit;
+        if (i < n_bins) {
+            k.bin[i] = i;
+            if (n > n_bins) {
+                heap.push_back({cost, i});
+                std::push_heap(heap.begin(), heap.end(), std::greater<Load>());
+            }
+            continue;
+        }
+        std::pop_heap(heap.begin(), heap.end(), std::greater<Load>());
+        k.bin[i] = heap.back().second;
+        heap.back().first += cost;
+        std::push_heap(heap.begin(), heap.end(), std::greater<Load>());
     }
-    return bins;
 }
 
-// Stream-K packing at capacity `cap`: blocks in the order largest,
-// smallest, second largest, second smallest, ... fill the bins in turn; a
-// block that does not fit is cut at the capacity and continues in the next
-// bin.  False when more than n_bins bins are needed.
-static bool stream_bins(const std::vector<std::pair<int, int>> &bt, double cap, int n_bins, const ScheduleCost &sc,
-                        Bins &bins) {
-    std::vector<int> order(bt.size());
-    for (size_t i = 0; i < order.size(); ++i) order[i] = (int)i;
-    std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
-        return bt[x].second - bt[x].first > bt[y].second - bt[y].first;
-    });
-    std::vector<int> seq;
-    for (int i = 0, j = (int)order.size() - 1; i <= j;) {
-        seq.push_back(order[i++]);
-        if (i <= j) seq.push_back(order[j--]);
-    }
-    bins.assign(1, {});
+// Stream-K packing at capacity `cap`: blocks in the order `seq` fill the bins
+// in turn; a block that does not fit is cut at the capacity and continues in
+// the next bin.  False when more than n_bins bins are needed.
+static bool stream_pack(const BlockTiles &bt, const std::vector<int> &seq, double cap, int n_bins,
+                        const ScheduleCost &sc, Packing &k) {
+    k.clear();
+    int bin = 0;
+    bool empty = true;
     double load = 0.0;
     for (int b : seq) {
         int lo = bt[b].first;
@@ -1424,11 +1443,11 @@ static bool stream_bins(const std::vector<std::pair<int, int>> &bt, double cap, 
         while (lo < hi) {
             const int rem = hi - lo;
             const double room = cap - load - sc.unit;
-            const bool empty = bins.back().empty();
             // An empty bin takes any remainder up to a minimum piece whole.
             if (rem <= room || (empty && rem <= kMinUnitTiles)) {
-                bins.back().push_back({b, lo, hi});
+                k.add(bin, {b, lo, hi});
                 load += rem + sc.unit;
+                empty = false;
                 break;
             }
             // The tiles that fit, leaving at least a minimum piece behind
@@ -1438,12 +1457,12 @@ static bool stream_bins(const std::vector<std::pair<int, int>> &bt, double cap, 
             if (rem - take < kMinUnitTiles) take = rem - kMinUnitTiles;
             if (empty) take = std::max(take, 1);
             if (take >= kMinUnitTiles || (empty && take >= 1)) {
-                bins.back().push_back({b, lo, lo + take});
+                k.add(bin, {b, lo, lo + take});
                 lo += take;
             }
             if (lo < hi) {
-                if ((int)bins.size() == n_bins) return false;
-                bins.push_back({});
+                if (++bin == n_bins) return false;
+                empty = true;
                 load = 0.0;
             }
         }
@@ -1451,49 +1470,63 @@ static bool stream_bins(const std::vector<std::pair<int, int>> &bt, double cap, 
     return true;
 }
 
-// The cheaper of the two schedules (by the cost model): fixed-length units
-// placed by LPT (16 .. 128 tiles, or longer when a block needs it to stay
-// within kPrefillMaxUnits units), or stream-K packing at the smallest
-// feasible capacity or a little above.  Stream-K wins on causal prompts
-// (every CU gets the same number of tiles, with about one split per CU);
-// LPT wins where few long blocks each need many pieces.
-static int build_schedule(const std::vector<std::pair<int, int>> &bt, int n_bins, const ScheduleCost &sc, Bins &best,
-                          int *slices) {
+// The cheapest schedule by the cost model: units of 1/k of the longest block
+// (k up to kPrefillMaxUnits) placed by LPT, or stream-K packing at the
+// smallest feasible capacity or a little above.  Stream-K wins on causal
+// prompts (every CU gets the same number of tiles, with about one split per
+// CU); LPT wins where few long blocks each need many pieces.  A prompt's
+// every chunk is a new shape, so this runs on the way to its first launch:
+// flat arrays and few candidates keep it at 0.04-0.2 ms (0.15-2 ms with nested
+// vectors, lengths in steps of 8 tiles and 12 capacities, at no better cost).
+static int build_schedule(const BlockTiles &bt, int n_bins, const ScheduleCost &sc, Bins &bins, int *slices) {
     int max_tiles = 1;
     long long total = 0;
     for (auto &x : bt) {
         max_tiles = std::max(max_tiles, x.second - x.first);
         total += x.second - x.first;
     }
-    double best_cost = -1.0;
-    auto consider = [&](Bins &&bins) {
-        int s = 1;
-        const double cost = schedule_cost(bins, (int)bt.size(), n_bins, sc, &s);
-        if (cost >= 0.0 && (best_cost < 0.0 || cost < best_cost)) {
-            best_cost = cost;
-            best = std::move(bins);
-            *slices = s;
-        }
+    Packing best, k;
+    ScheduleScratch tmp;
+    auto consider = [&] {
+        price(k, (int)bt.size(), n_bins, sc, tmp);
+        if (k.cost >= 0.0 && (best.cost < 0.0 || k.cost < best.cost)) std::swap(best, k);
     };
-    const int ut_hi = std::max(128, ((max_tiles + kPrefillMaxUnits - 1) / kPrefillMaxUnits + 7) / 8 * 8);
-    for (int ut = ut_hi; ut >= 16; ut -= 8) {
-        if ((max_tiles + ut - 1) / ut > kPrefillMaxUnits) break;
-        consider(lpt_bins(bt, ut, n_bins, sc));
+    for (int n = 1, last = 0; n <= kPrefillMaxUnits; ++n) {
+        const int ut = std::max(kMinUnitTiles, (max_tiles + n - 1) / n);
+        // (Four small pieces per workgroup balance as well as eight.)
+        if (ut == last || (n > 1 && (int)bt.size() * n > 4 * n_bins)) break;
+        last = ut;
+        lpt_pack(bt, ut, n_bins, sc, k);
+        consider();
+    }
+    // Largest, smallest, second largest, second smallest, ...
+    std::vector<int> order(bt.size()), seq;
+    for (size_t i = 0; i < order.size(); ++i) order[i] = (int)i;
+    std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
+        return bt[x].second - bt[x].first > bt[y].second - bt[y].first;
+    });
+    seq.reserve(bt.size());
+    for (int i = 0, j = (int)order.size() - 1; i <= j;) {
+        seq.push_back(order[i++]);
+        if (i <= j) seq.push_back(order[j--]);
     }
     double lo = (double)total / n_bins + sc.unit, hi = lo + max_tiles + 2 * sc.unit;
-    Bins bins;
-    if (stream_bins(bt, hi, n_bins, sc, bins)) {
-        while (hi - lo > 0.25) {
+    if (stream_pack(bt, seq, hi, n_bins, sc, k)) {
+        while (hi - lo > 0.5) {
             const double mid = 0.5 * (lo + hi);
-            if (stream_bins(bt, mid, n_bins, sc, bins))
+            if (stream_pack(bt, seq, mid, n_bins, sc, k))
                 hi = mid;
             else
                 lo = mid;
         }
-        for (int k = 0; k < 12; ++k)
-            if (stream_bins(bt, hi + 0.5 * k, n_bins, sc, bins)) consider(std::move(bins));
+        for (int i = 0; i < 6; ++i)
+            if (stream_pack(bt, seq, hi + i, n_bins, sc, k)) consider();
     }
-    return best_cost < 0.0 ? -1 : 0;
+    if (best.cost < 0.0) return -1;
+    bins.assign(best.used, {});
+    for (size_t i = 0; i < best.pieces.size(); ++i) bins[best.bin[i]].push_back(best.pieces[i]);
+    *slices = best.slices;
+    return 0;
 }
 
 // The unit table, workgroup ranges and block table of a schedule; checks
@@ -1601,32 +1634,45 @@ static int plan_for(g4_ctx *ctx, const PrefillArgs &a, bool split, const Prefill
     pl.n_blocks = (int)blocks.size();
     pl.n_slots = n_slots;
     pl.last_use = ps.tick;
-    hipError_t e = hipMalloc(&pl.units, units.size() * sizeof(PrefillUnit));
-    if (e == hipSuccess) e = hipMalloc(&pl.bin_start, bin_start.size() * sizeof(int));
-    if (e == hipSuccess) e = hipMalloc(&pl.blocks, blocks.size() * sizeof(PrefillBlockInfo));
-    if (e == hipSuccess)
-        e = hipMemcpy(pl.units, units.data(), units.size() * sizeof(PrefillUnit), hipMemcpyHostToDevice);
-    if (e == hipSuccess)
-        e = hipMemcpy(pl.bin_start, bin_start.data(), bin_start.size() * sizeof(int), hipMemcpyHostToDevice);
-    if (e == hipSuccess)
-        e = hipMemcpy(pl.blocks, blocks.data(), blocks.size() * sizeof(PrefillBlockInfo), hipMemcpyHostToDevice);
-    if (e != hipSuccess) {
-        free_plan(pl);
-        return hip_failed(e, "prefill unit table");
-    }
-    if (ps.plans.size() >= kPrefillPlans) {
-        size_t lru = 0;
+    // One image of the tables, one copy.
+    const size_t ub = units.size() * sizeof(PrefillUnit), bb = blocks.size() * sizeof(PrefillBlockInfo);
+    std::vector<char> image(ub + bb + bin_start.size() * sizeof(int));
+    memcpy(image.data(), units.data(), ub);
+    memcpy(image.data() + ub, blocks.data(), bb);
+    memcpy(image.data() + ub + bb, bin_start.data(), bin_start.size() * sizeof(int));
+    size_t at = ps.plans.size();
+    if (at >= kPrefillPlans) {
+        at = 0;
         for (size_t i = 1; i < ps.plans.size(); ++i)
-            if (ps.plans[i].last_use < ps.plans[lru].last_use) lru = i;
+            if (ps.plans[i].last_use < ps.plans[at].last_use) at = i;
         // Kernels on any stream may still read the evicted table.
         G4_HIP(hipDeviceSynchronize());
-        free_plan(ps.plans[lru]);
-        ps.plans[lru] = pl;
-        *out = &ps.plans[lru];
+        std::swap(pl.mem, ps.plans[at].mem);
+        std::swap(pl.mem_bytes, ps.plans[at].mem_bytes);
+        ps.plans[at].pos0 = -1;  // no shape's table until the new one is in
     } else {
-        ps.plans.push_back(pl);
-        *out = &ps.plans.back();
+        ps.plans.emplace_back();
     }
+    PrefillPlan &slot = ps.plans[at];
+    hipError_t e = hipSuccess;
+    if (pl.mem_bytes < image.size()) {
+        if (pl.mem) (void)hipFree(pl.mem);
+        pl.mem = nullptr;
+        pl.mem_bytes = 0;
+        e = hipMalloc(&pl.mem, image.size());
+        if (e == hipSuccess) pl.mem_bytes = image.size();
+    }
+    if (e == hipSuccess) e = hipMemcpy(pl.mem, image.data(), image.size(), hipMemcpyHostToDevice);
+    if (e != hipSuccess) {
+        slot.mem = pl.mem;
+        slot.mem_bytes = pl.mem_bytes;
+        return hip_failed(e, "prefill unit table");
+    }
+    pl.units = (PrefillUnit *)pl.mem;
+    pl.blocks = (PrefillBlockInfo *)((char *)pl.mem + ub);
+    pl.bin_start = (int *)((char *)pl.mem + ub + bb);
+    slot = pl;
+    *out = &slot;
     return G4_OK;
 }
 

@@ -185,3 +185,23 @@ def test_prefill_schedule_forms(ctx, pos0, N, window, d):
     for i in rows:
         b, e = I.attended_range(pos0 + i, window)
         assert I.rel_err(got[i], orc.attend(q[pos0 + i], K[b:e], V[b:e], 8, 1)) <= TOL, i
+
+
+def test_prefill_more_shapes_than_the_context_keeps(ctx):
+    """More shapes in turn than the context keeps schedules for (128), twice
+    over: the second pass, which rebuilds the evicted tables in their
+    memory, gives the first one's bits, and those match the oracle."""
+    d, N, shapes = 256, 11, 140
+    q, K, V = case(5, shapes + N, d, False)
+    outs = []
+    for again in range(2):
+        for pos0 in range(shapes):
+            got = prefill(ctx, q[pos0:pos0 + N], K, V, pos0, N, 100, d)
+            if again:
+                assert np.array_equal(got, outs[pos0]), pos0
+            else:
+                outs.append(got)
+    for pos0 in (0, 77, shapes - 1):
+        for i in range(N):
+            b, e = I.attended_range(pos0 + i, 100)
+            assert I.rel_err(outs[pos0][i], orc.attend(q[pos0 + i], K[b:e], V[b:e], 8, 1)) <= TOL
