@@ -105,3 +105,27 @@ def test_ragged_decode_split_sizes(ctx, d, B, bound):
     lens[B // 2] = bound
     print(f"[case] ragged splits d={d} B={B} bound={bound}", flush=True)
     test_ragged_decode_random_batches(ctx, d, 0, lens.tolist())
+
+
+@pytest.mark.parametrize("d,bound", [(256, 512), (512, 250), (256, 130)])
+def test_ragged_decode_after_non_finite_partials(ctx, d, bound):
+    """The merge reads split slots past a short sequence's count: left full
+    of NaN by an earlier batch, they must not reach its output."""
+    B = 6
+    K = np.random.default_rng(d).standard_normal((B * bound, d), dtype=np.float32) * 0.1
+    V = np.full((B * bound, d), np.nan, np.float32)
+    q = np.random.default_rng(bound).standard_normal((B, 8 * d), dtype=np.float32) * 0.1
+    row0 = np.arange(B, dtype=np.int64) * bound
+    begin = np.zeros(B, np.int64)
+    out = torch.zeros(B * 8 * d, device="cuda")
+    ctx.attend_decode_batch(dev(q), dev(K), dev(V), dev(row0), dev(begin), dev(begin + bound), bound, 8, 1, d, out)
+    torch.cuda.synchronize()
+    assert torch.isnan(out).all()
+    V = np.random.default_rng(3).standard_normal((B * bound, d), dtype=np.float32)
+    lens = np.array([1, 17, 33, bound // 2, bound - 1, bound], np.int64)
+    ctx.attend_decode_batch(dev(q), dev(K), dev(V), dev(row0), dev(begin), dev(lens), bound, 8, 1, d, out)
+    ctx.check_status()
+    got = out.cpu().numpy().reshape(B, -1)
+    for s in range(B):
+        rows = slice(row0[s], row0[s] + lens[s])
+        assert I.rel_err(got[s], orc.attend(q[s], K[rows], V[rows], 8, 1)) <= TOL
