@@ -160,8 +160,13 @@ __global__ __launch_bounds__(64) void matvec_q8_0_kernel(const unsigned char *__
     for (int s = 0; s < NS; ++s) {
         const int b = lane + 64 * s;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) xqr[s][j] = b < nb ? xq[b * 8 + j] : 0;
-        xsr[s] = b < nb ? xs[b] : 0.0f;
+        for (int j = 0; j < 8; ++j) xqr[s][j] = 0;
+        xsr[s] = 0.0f;
+        if (b < nb) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) xqr[s][j] = xq[b * 8 + j];
+            xsr[s] = xs[b];
+        }
     }
 
     for (int r0 = 0; r0 < n_rows; r0 += g) {
@@ -303,7 +308,7 @@ __device__ inline void stage_activation(float *act, int nb, const float *xs, con
 }
 
 // W @ x for Q8_0 rows, the matrices that do not fill the chip for long
-// (everything but the output head).  They are bound by one trip to memory,
+// (everything but a whole output head).  They are bound by one trip to memory,
 // so every byte is asked for at once: about one workgroup per CU, whose nw
 // row wavefronts each bring rw consecutive rows (one run of bytes, per
 // matrix) into LDS with 16-byte direct-to-LDS loads, while nq further
@@ -713,8 +718,10 @@ int launch_q8_once(g4_ctx *ctx, const MatvecArgs &a, hipStream_t stream, bool *d
     if (nb64 <= 0 || nb64 > 8192 || (uintptr_t)a.w % 4 != 0 || (NM == 2 && (uintptr_t)a.w2 % 4 != 0)) return G4_OK;
     const int nb = (int)nb64;
     // One workgroup per CU with a row wavefront per row, up to 8, then more
-    // rows per wavefront; where that does not fit a CU's LDS, two workgroups
-    // per CU, each within half of it.
+    // rows per wavefront.  Where that does not fit a CU's LDS, rounds of
+    // smaller workgroups, of 4 row wavefronts and five to a CU, whose loads,
+    // products and sums overlap (84,752 x 768 17.2 us, 49,152 x 1536 17.8;
+    // 8 wavefronts and two to a CU 20.9 and 20.0; three 17.8 and 20.1).
     constexpr size_t kLds = 160 * 1024;
     auto bytes = [&](int nw, int rw) {
         const Q8OnceLds at(nb, rw, NM, kValue, kActBlock<DOT>);
@@ -723,8 +730,9 @@ int launch_q8_once(g4_ctx *ctx, const MatvecArgs &a, hipStream_t stream, bool *d
     const int64_t per_cu = std::min<int64_t>(8 * (64 / NM), (a.rows + ctx->num_cus - 1) / ctx->num_cus);
     int nw = (int)std::min<int64_t>(8, per_cu), rw = (int)((per_cu + nw - 1) / nw);
     if (bytes(nw, rw) > kLds) {
-        while (rw > 1 && bytes(nw, rw) > kLds / 2) --rw;
-        while (nw > 1 && bytes(nw, rw) > kLds / 2) --nw;
+        nw = std::min(nw, 4);
+        while (rw > 1 && bytes(nw, rw) > kLds / 5) --rw;
+        while (nw > 1 && bytes(nw, rw) > kLds / 5) --nw;
         if (bytes(nw, rw) > kLds) return G4_OK;
     }
     const int nq = std::min(4, (nb + 23) / 24);
@@ -750,7 +758,13 @@ int launch_q8(g4_ctx *ctx, MatvecArgs a, hipStream_t stream) {
     const bool staged = a.cols % 256 == 0 && nb > 0 && nb <= 256 && aligned;
     // Rows per workgroup: up to 16, the product table under 16 KB.
     const int64_t rb_max = std::min<int64_t>(16, std::max<int64_t>(1, 16384 / (NM * (nb + 1) * 4)));
-    const bool large = staged && a.rows >= rb_max * 8 * num_cus;
+    // The streaming kernel, which needs its activation quantized by a launch
+    // of its own, pays from some 128 MB on: 33,017 x 1024 (36 MB) 13.3 us
+    // against 11.0 at once, 84,752 x 768 (69 MB) 20.4 against 17.2, 131,072 x
+    // 1280 (178 MB) 35.3 against 35.0, the output head (429 MB) 71.0 against
+    // 72.1.
+    const bool large = staged && a.rows >= rb_max * 8 * num_cus &&
+                       a.rows * nb * kQ8Bytes * NM > (512LL << 10) * num_cus;
     if (!large) {
         bool done = false;
         const int rc = launch_q8_once<EPI, kInt8>(ctx, a, stream, &done);
