@@ -971,10 +971,8 @@ __device__ __forceinline__ void merge_fold(const DecodeK &p, int64_t slot0, int6
 // split count n is uniform in the workgroup: the batch size is the smallest
 // that covers n in one memory round trip (up to 256 splits), so no lane
 // reloads a split it does not use.
-// Four wavefronts per SIMD (128 VGPRs): the 32-sequence batch's 1024
-// workgroups are resident at once.
 template <int MODE, int D, int EPW>
-__global__ __launch_bounds__(256, 4) void decode_merge_kernel(DecodeK p) {
+__global__ __launch_bounds__(256) void decode_merge_kernel(DecodeK p) {
     constexpr int PH = 256 / EPW;
     static_assert(EPW == 8 || EPW == 16, "whole 128-byte rows per phase; at most 16 lanes write");
     const int s = blockIdx.z, kvh = blockIdx.y;
@@ -1041,7 +1039,9 @@ __global__ __launch_bounds__(256, 4) void decode_merge_kernel(DecodeK p) {
         merge_fold<D, PH, 2>(p, slot0, jslot, first_extra, ph, e, c, n, G, mt, lt, ot);
     else if (n <= 4 * PH)
         merge_fold<D, PH, 4>(p, slot0, jslot, first_extra, ph, e, c, n, G, mt, lt, ot);
-    else if (n <= 8 * PH || EPW == 8)
+    else if (n <= 8 * PH || EPW == 8 || MODE == kBatch || MODE == kPrefill)
+        // Batches of sequences have few splits each and many workgroups,
+        // which keep four wavefronts per SIMD without the widest batch.
         merge_fold<D, PH, 8>(p, slot0, jslot, first_extra, ph, e, c, n, G, mt, lt, ot);
     else
         merge_fold<D, PH, 16>(p, slot0, jslot, first_extra, ph, e, c, n, G, mt, lt, ot);
