@@ -707,8 +707,8 @@ int launch_q8_rows(const MatvecArgs &a, int g, int rb, hipStream_t stream) {
 }
 
 // Launches matvec_q8_0_once_kernel, or says (*done) that the shape does not
-// suit it: a matrix off a 4-byte boundary, no blocks, or rows too long for a
-// CU's LDS.
+// suit it: a matrix off a 4-byte boundary, no blocks, rows too long for a
+// CU's LDS, or more workgroups than a launch takes.
 template <int EPI, int DOT>
 int launch_q8_once(g4_ctx *ctx, const MatvecArgs &a, hipStream_t stream, bool *done) {
     constexpr int NM = EPI >= kGeglu ? 2 : 1;
@@ -737,7 +737,7 @@ int launch_q8_once(g4_ctx *ctx, const MatvecArgs &a, hipStream_t stream, bool *d
     }
     const int nq = std::min(4, (nb + 23) / 24);
     const int64_t groups = (a.rows + (int64_t)nw * rw - 1) / ((int64_t)nw * rw);
-    if (groups >= (1LL << 31)) return G4_OK;
+    if (groups > (1LL << 22)) return G4_OK;  // a launch holds fewer than 2^32 threads
     hipLaunchKernelGGL((matvec_q8_0_once_kernel<EPI, DOT>), dim3((unsigned)groups), dim3(64 * (nw + nq)),
                        bytes(nw, rw), stream, a.w, a.w2, a.rows, nb, DOT == kInt8 ? a.xs : nullptr,
                        (const int *)a.xq, a.x, a.arg, nw, nq, rw, a.out);
@@ -815,9 +815,13 @@ int launch_q8_f32(g4_ctx *ctx, const MatvecArgs &a, hipStream_t stream) {
 
 template <typename W, int R, int P, bool VEC>
 int launch_dense_rows(const MatvecArgs &a, hipStream_t stream) {
-    hipLaunchKernelGGL((matvec_dense_kernel<W, R, P, VEC>), dim3((unsigned)((a.rows + R - 1) / R)), dim3(128), 0,
-                       stream, (const W *)a.w, a.rows, a.cols, a.x, a.out);
-    G4_HIP(hipGetLastError());
+    constexpr int64_t kRows = (int64_t)R << 24;  // a launch holds fewer than 2^32 threads
+    for (int64_t r0 = 0; r0 < a.rows; r0 += kRows) {
+        const int64_t rows = std::min(kRows, a.rows - r0);
+        hipLaunchKernelGGL((matvec_dense_kernel<W, R, P, VEC>), dim3((unsigned)((rows + R - 1) / R)), dim3(128), 0,
+                           stream, (const W *)a.w + r0 * a.cols, rows, a.cols, a.x, a.out + r0);
+        G4_HIP(hipGetLastError());
+    }
     return G4_OK;
 }
 

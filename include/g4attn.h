@@ -160,7 +160,9 @@ int g4_attend_prefill(g4_ctx *ctx, const float *q_dev, const float *k_cache_dev,
  * (of n_bins per KV head) runs units bin_start[w] .. bin_start[w+1]-1 in
  * turn.  units (host) gets 4 int32 per unit: {block, first tile, end tile,
  * partial slot or -1 for a block computed by one unit}; bin_start (host)
- * n_bins+1 entries; counts (host) {n_units, n_bins, n_slots}.  Host only,
+ * n_bins+1 entries; counts (host) {n_units, n_bins, n_slots}.  Where the bins
+ * do not fill the GPU, a unit's tiles are shared out further, over several
+ * workgroups that each leave a partial (not listed here).  Host only,
  * no device work; counts are filled even when the arrays are too small
  * (then G4_ERR_MSG).  No counterpart in the reference, whose prompt runs
  * token at a time (crates/llm-gemma4/src/impl_/generate.rs:37-41). */
