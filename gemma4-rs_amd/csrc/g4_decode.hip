@@ -22,7 +22,7 @@
 // S^T over its dims; the partials are summed through LDS in a fixed order, so
 // every wave sees bit-identical scores and softmax state, then each wave
 // accumulates P.V for its own dims.  Work is split over keys (split-K): a
-// workgroup handles a power-of-two run of keys of one (sequence, KV head),
+// workgroup handles a run of whole 16-key tiles of one (sequence, KV head),
 // streaming 16-key tiles through a ring of register buffers (loads of the
 // next tiles in flight while the current one is computed), and leaves an
 // online-softmax partial (m, l, O) that a second kernel merges.

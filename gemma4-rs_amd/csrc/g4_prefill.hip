@@ -26,9 +26,10 @@
 // tiles than the first, so a block's key range may be cut into units (at
 // most kPrefillMaxUnitsDev per block), and the host assigns every unit to a
 // workgroup (at most one per CU), which runs its units in turn; the
-// schedule builder below explains the choice.  A block with one unit writes
-// its output directly; otherwise each unit leaves an (m, l, O) partial and a
-// merge kernel combines them in key order.
+// schedule builder below explains the choice; where the units do not fill
+// the chip, several workgroups share each unit's tiles.  A block with one
+// unit, run by one workgroup, writes its output directly; otherwise each
+// piece leaves an (m, l, O) partial and a merge kernel combines them.
 
 #include <algorithm>
 #include <cmath>
@@ -36,7 +37,6 @@
 #include <climits>
 #include <cstring>
 #include <functional>
-#include <queue>
 #include <utility>
 #include <vector>
 

@@ -66,6 +66,23 @@ def test_schedule_covers_every_attended_tile_once(pos0, N, window, d, n_kv):
     assert sorted(all_slots) == list(range(len(all_slots)))
 
 
+def _drawn_shapes():
+    rng = np.random.default_rng(77)
+    out = []
+    for _ in range(40):
+        d = int(rng.choice([256, 512]))
+        window = int(rng.choice([0, 1, 17, 512, 4096]))
+        N, pos0 = int(2 ** rng.uniform(0, 11.5)), int(rng.choice([0, 2 ** rng.uniform(0, 15)]))
+        out.append((pos0, N, window, d, int(rng.choice([1, 1, 2, 4]))))
+    return out
+
+
+@pytest.mark.parametrize("pos0,N,window,d,n_kv", _drawn_shapes())
+def test_schedule_of_drawn_shapes(pos0, N, window, d, n_kv):
+    """The same over drawn shapes, windows and KV head counts."""
+    test_schedule_covers_every_attended_tile_once(pos0, N, window, d, n_kv)
+
+
 def bin_tiles(units, bins):
     return np.array([int((units[bins[w]:bins[w + 1], 2] - units[bins[w]:bins[w + 1], 1]).sum())
                      for w in range(len(bins) - 1)])
