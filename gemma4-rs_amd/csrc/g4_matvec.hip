@@ -322,10 +322,10 @@ __device__ inline void stage_activation(float *act, int nb, const float *xs, con
 // bytes (fewer than 16) as 2-byte values.
 // Weights from HBM, activation as f32 (one wavefront per two or three rows
 // that quantized the activation for itself, before -> here): 2048 x 1536
-// 5.4 -> 4.0 us, 4096 x 1536 6.3 -> 5.0, 1536 x 6144 11.3 -> 7.5, gate and up
-// of 6144 x 1536 (20.9 MB) 10.3 -> 7.7; a plain read of 16 MiB takes 4.7.
+// 5.4 -> 4.0 us, 4096 x 1536 6.3 -> 5.0, 1536 x 6144 11.3 -> 7.1, gate and up
+// of 6144 x 1536 (20.9 MB) 10.3 -> 7.6; a plain read of 16 MiB takes 4.7.
 // f32 activations, one lane per row before: 2048 x 1536 27 -> 3.8 us,
-// 1536 x 6144 172 -> 7.4.
+// 1536 x 6144 172 -> 7.0.
 template <int EPI, int DOT>
 __global__ __launch_bounds__(768) void matvec_q8_0_once_kernel(const unsigned char *__restrict__ w,
                                                                const unsigned char *__restrict__ w2, int64_t rows,
@@ -421,24 +421,32 @@ __global__ __launch_bounds__(768) void matvec_q8_0_once_kernel(const unsigned ch
                 }
             }
     }
-    // Lane m*rw + r sums row r of matrix m, 16 products read ahead.
+    // Lane m*rw + r sums row r of matrix m, 16 products at a time with the
+    // next 32 on their way: 16 adds are shorter than an LDS read (1536 x
+    // 6144 with only 16 ahead 7.5 us, 7.1 so; five layers' calls 167.7 ->
+    // 163.2).
     T sum = (T)-0.0;
     if (lane < NM * rw) {
         const vec *pr = (const vec *)(prod + lane * at.pstride);
-        vec cur[16 / V], nxt[16 / V];
+        const int groups = at.padded / 16;
+        vec v[3][16 / V];
+        auto read = [&](int g, vec (&dst)[16 / V]) {
 #pragma unroll
-        for (int i = 0; i < 16 / V; ++i) cur[i] = pr[i];
-        for (int b = 16; b <= at.padded; b += 16) {
-            const int ahead = min(b, at.padded - 16) / V;
+            for (int i = 0; i < 16 / V; ++i) dst[i] = pr[min(g, groups - 1) * (16 / V) + i];
+        };
+        read(0, v[0]);
+        read(1, v[1]);
+        for (int g = 0; g < groups; g += 3) {
 #pragma unroll
-            for (int i = 0; i < 16 / V; ++i) nxt[i] = pr[ahead + i];
-            __builtin_amdgcn_sched_barrier(0);
+            for (int p = 0; p < 3; ++p) {
+                if (g + p >= groups) break;
+                read(g + p + 2, v[(p + 2) % 3]);
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int i = 0; i < 16 / V; ++i)
+                for (int i = 0; i < 16 / V; ++i)
 #pragma unroll
-                for (int k = 0; k < V; ++k) sum += cur[i][k];
-#pragma unroll
-            for (int i = 0; i < 16 / V; ++i) cur[i] = nxt[i];
+                    for (int k = 0; k < V; ++k) sum += v[p][i][k];
+            }
         }
     }
     float v = (float)sum;
