@@ -182,7 +182,8 @@ __device__ inline void combine_partial(float &m, float &l, f32x4 &o, float m2, f
 }
 
 // Folds a batch of split partials (m_j, l_j) / O_j into the running
-// (m, l, o) of one stored vector; entries at or past n are ignored.
+// (m, l, o) of one stored vector.  Entries at or past n get a weight of 0:
+// they must hold finite l and O (another split's, or an empty partial).
 template <int NB>
 __device__ inline void fold_batch(float &m, float &l, f32x4 &o, const float2 (&t)[NB], const f32x4 (&v)[NB],
                                   int j0, int jstep, int n) {
@@ -1001,11 +1002,13 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(DecodeK p) {
     } else if constexpr (MODE != kSingle) {
         // How many splits a sequence has takes a trip to memory for its
         // range.  Where at most two loads per phase cover the most that any
-        // sequence can have, they go out beside the range's: a slot past the
-        // count holds whatever the workspace held, and is dropped.  (8
-        // ragged sequences through 35 layers as a graph: 402 -> 393 us.)
-        // With few splits the batch has many sequences, whose workgroups
-        // cover for each other's trip (32 x 512 keys: no gain).
+        // sequence can have, they go out beside the range's.  A slot past
+        // the count holds whatever the workspace held, NaN and infinities
+        // included, which a weight of 0 would not keep out of a sum: it is
+        // replaced by an empty partial.  (8 ragged sequences through 35
+        // layers as a graph: 402 -> 393 us.)  With few splits the batch has
+        // many sequences, whose workgroups cover for each other's trip (32 x
+        // 512 keys: no gain).
         float2 t[2] = {float2{-INFINITY, 0.0f}, float2{-INFINITY, 0.0f}};
         f32x4 v[2] = {};
         folded = n > PH / 2 && n <= 2 * PH;
@@ -1026,7 +1029,10 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(DecodeK p) {
         if (folded) {
 #pragma unroll
             for (int b = 0; b < 2; ++b)
-                if (ph + PH * b >= n) v[b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                if (ph + PH * b >= n) {
+                    t[b] = float2{-INFINITY, 0.0f};
+                    v[b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                }
             fold_batch(mt, lt, ot, t, v, ph, PH, n);
         }
     }

@@ -129,3 +129,92 @@ def test_ragged_decode_after_non_finite_partials(ctx, d, bound):
     for s in range(B):
         rows = slice(row0[s], row0[s] + lens[s])
         assert I.rel_err(got[s], orc.attend(q[s], K[rows], V[rows], 8, 1)) <= TOL
+
+
+def _poison_and_check(ctx, d, poison, K, V, q, bound, lens, row0):
+    """poison() leaves its partials in the workspace and fails its own status
+    check; the batch over `lens` that follows must not see them."""
+    import g4hip
+    poison()
+    with pytest.raises(g4hip.EngError):
+        ctx.check_status()
+    B = len(lens)
+    out = torch.zeros(B * 8 * d, device="cuda")
+    begin = np.zeros(B, np.int64)
+    ctx.attend_decode_batch(dev(q), dev(K), dev(V), dev(row0), dev(begin), dev(lens), bound, 8, 1, d, out)
+    ctx.check_status()
+    got = out.cpu().numpy().reshape(B, -1)
+    for s in range(B):
+        rows = slice(row0[s], row0[s] + lens[s])
+        assert I.rel_err(got[s], orc.attend(q[s], K[rows], V[rows], 8, 1)) <= TOL, s
+
+
+@pytest.mark.parametrize("value", [np.nan, 1e38])
+@pytest.mark.parametrize("d,bound", [(256, 135), (256, 250), (512, 144), (256, 260), (512, 400), (512, 512)])
+def test_ragged_decode_after_non_finite_softmax_sums(ctx, d, bound, value):
+    """9 to 32 split slots per sequence, each left with a NaN maximum or sum
+    by a batch whose keys hold NaN, or overflow their scores: a shorter
+    sequence in the slot's place must not see them.  (Splits are 16 keys.)"""
+    B = 6
+    rng = np.random.default_rng(d + bound)
+    K = rng.standard_normal((B * bound, d), dtype=np.float32) * 0.1
+    V = rng.standard_normal((B * bound, d), dtype=np.float32)
+    q = rng.standard_normal((B, 8 * d), dtype=np.float32) * 0.1
+    row0 = np.arange(B, dtype=np.int64) * bound
+    bad = K.copy()
+    bad[::5] = value  # every split holds some
+    hot = np.full_like(q, 50.0)
+    ends = np.full(B, bound, np.int64)
+    out = torch.zeros(B * 8 * d, device="cuda")
+    lens = np.array([1, 17, 33, bound // 2, bound - 17, bound], np.int64)
+    _poison_and_check(ctx, d, lambda: ctx.attend_decode_batch(dev(hot), dev(bad), dev(V), dev(row0), dev(ends * 0),
+                                                              dev(ends), bound, 8, 1, d, out),
+                      K, V, q, bound, lens, row0)
+
+
+@pytest.mark.parametrize("d", [256, 512])
+def test_ragged_decode_over_another_bounds_outputs(ctx, d):
+    """A batch with a larger bound leaves NaN outputs where a later batch's
+    (m, l) pairs lie."""
+    B, wide, bound = 6, 512, 200
+    rng = np.random.default_rng(d)
+    K = rng.standard_normal((B * wide, d), dtype=np.float32) * 0.1
+    V = rng.standard_normal((B * wide, d), dtype=np.float32)
+    q = rng.standard_normal((B, 8 * d), dtype=np.float32) * 0.1
+    row0 = np.arange(B, dtype=np.int64) * wide
+    ends = np.full(B, wide, np.int64)
+    bad = K.copy()
+    bad[::16] = np.nan
+    nan_v = np.full_like(V, np.nan)
+    out = torch.zeros(B * 8 * d, device="cuda")
+    lens = np.array([1, 17, 33, bound // 2, bound - 17, bound], np.int64)
+    _poison_and_check(ctx, d, lambda: ctx.attend_decode_batch(dev(q), dev(bad), dev(nan_v), dev(row0), dev(ends * 0),
+                                                              dev(ends), wide, 8, 1, d, out),
+                      K, V, q, bound, lens, row0)
+
+
+@pytest.mark.parametrize("chunk,pos0,N", [(0, 890, 40), (16, 0, 300)])
+def test_generic_prefill_after_non_finite_softmax_sums(ctx, chunk, pos0, N):
+    """The same through a prompt chunk of a shape outside the MFMA prefill (4
+    heads on one KV head), whose queries have different split counts."""
+    import g4hip
+    d, heads = 256, 4
+    rng = np.random.default_rng(pos0 + N)
+    K = rng.standard_normal((pos0 + N, d), dtype=np.float32) * 0.1
+    V = rng.standard_normal((pos0 + N, d), dtype=np.float32)
+    q = rng.standard_normal((N, heads * d), dtype=np.float32) * 0.1
+    out = torch.zeros(N * heads * d, device="cuda")
+    ctx.set_decode_chunk(chunk)
+    try:
+        bad = K.copy()
+        bad[::5] = np.nan
+        ctx.attend_prefill(dev(q), dev(bad), dev(V), pos0, N, 0, heads, 1, d, out)
+        with pytest.raises(g4hip.EngError):
+            ctx.check_status()
+        ctx.attend_prefill(dev(q), dev(K), dev(V), pos0, N, 0, heads, 1, d, out)
+        ctx.check_status()
+    finally:
+        ctx.set_decode_chunk(0)
+    got = out.cpu().numpy().reshape(N, -1)
+    for i in range(N):
+        assert I.rel_err(got[i], orc.attend(q[i], K[:pos0 + i + 1], V[:pos0 + i + 1], heads, 1)) <= TOL, i
