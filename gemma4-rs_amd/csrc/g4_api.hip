@@ -50,6 +50,16 @@ int hip_failed(hipError_t e, const char *what) {
     return set_error(G4_ERR_COMPUTE, std::string("hip: ") + hipGetErrorString(e) + " (" + what + ")");
 }
 
+bool capturing(hipStream_t stream) {
+    if (!stream) return false;  // the null stream cannot be captured
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &st) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return st == hipStreamCaptureStatusActive;
+}
+
 int ensure_workspace(g4_ctx *ctx, size_t bytes, hipStream_t stream) {
     (void)stream;
     if (ctx->ws.bytes >= bytes) return G4_OK;

@@ -46,12 +46,16 @@ struct g4_ctx {
     int num_cus = 256;
     int64_t *zero_rows = nullptr;    // device zeros: default row offsets of a batch
     int64_t zero_rows_len = 0;
-    void *prefill_plan = nullptr;    // work-unit table of the last prefill shape
+    void *prefill_plan = nullptr;    // work-unit tables of the last prefill shapes
     void *scratch = nullptr;         // this device's static decode scratch (g4_attend_decode_noalloc)
     size_t scratch_bytes = 0;
 };
 
 namespace g4 {
+
+// Whether work launched on `stream` is being recorded into a graph, which
+// will use the same buffers at any later time.
+bool capturing(hipStream_t stream);
 
 // Grows the context's workspace to at least `bytes` (stream-ordered users
 // must not be in flight on another stream when it grows).

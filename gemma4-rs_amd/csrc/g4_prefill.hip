@@ -1307,15 +1307,17 @@ struct PrefillPlan {
     PrefillBlockInfo *blocks = nullptr;
     PrefillBin *bins = nullptr;
     uint64_t last_use = 0;
+    bool captured = false;  // a graph holds its address: never evicted
 };
 
 // The context's tables for the last shapes.  A layer-by-layer prompt alternates
 // sliding and global shapes, two new ones per chunk, and comes back to them for
 // every prompt of its chunk size: 64 chunks' tables (10 KB or so each) stay.
 // With 8, a 2048-token prompt in chunks of 256 rebuilt every table on every
-// pass (2.2 ms for one layer of each kind).  A cached table is never written
-// again, so kernels still in flight on any stream keep reading a valid table;
-// only evicting one waits for the device.
+// pass (2.2 ms for one layer of each kind).  Evicting a table rewrites its
+// memory for another shape, after a wait for kernels in flight on any stream.
+// A graph that was captured with a table reads it at every replay, so such a
+// table stays until the context goes, and does not count among the 128.
 constexpr size_t kPrefillPlans = 128;
 struct PrefillPlans {
     std::vector<PrefillPlan> plans;
@@ -1630,13 +1632,14 @@ static int bins_for(int num_cus, int n_kv_heads) { return std::max(1, num_cus / 
 
 // The schedule tables of a's shape: cached, or built and uploaded
 // (synchronously: graph capture needs an earlier call with the same shape).
-static int plan_for(g4_ctx *ctx, const PrefillArgs &a, bool split, const PrefillPlan **out) {
+static int plan_for(g4_ctx *ctx, const PrefillArgs &a, bool split, hipStream_t stream, const PrefillPlan **out) {
     PrefillPlans &ps = plans_of(ctx);
     ++ps.tick;
     for (auto &pl : ps.plans)
         if (pl.pos0 == a.pos0 && pl.N == a.N && pl.window == a.window && pl.head_dim == a.head_dim &&
             pl.n_kv_heads == a.n_kv_heads && pl.split == split) {
             pl.last_use = ps.tick;
+            pl.captured |= capturing(stream);
             *out = &pl;
             return G4_OK;
         }
@@ -1674,6 +1677,7 @@ static int plan_for(g4_ctx *ctx, const PrefillArgs &a, bool split, const Prefill
     pl.n_blocks = (int)blocks.size();
     pl.n_slots = n_slots;
     pl.last_use = ps.tick;
+    pl.captured = capturing(stream);
     // One image of the tables, one copy.
     std::vector<PrefillBin> table(pl.n_bins);
     for (int b = 0; b < pl.n_bins; ++b) table[b] = {bin_start[b], bin_start[b + 1], {0, 0}, units[bin_start[b]]};
@@ -1683,18 +1687,20 @@ static int plan_for(g4_ctx *ctx, const PrefillArgs &a, bool split, const Prefill
     memcpy(image.data(), table.data(), tb);
     memcpy(image.data() + tb, units.data(), ub);
     memcpy(image.data() + tb + ub, blocks.data(), bb);
-    size_t at = ps.plans.size();
-    if (at >= kPrefillPlans) {
-        at = 0;
-        for (size_t i = 1; i < ps.plans.size(); ++i)
-            if (ps.plans[i].last_use < ps.plans[at].last_use) at = i;
+    size_t at = ps.plans.size(), evictable = 0;
+    for (size_t i = 0; i < ps.plans.size(); ++i) {
+        if (ps.plans[i].captured) continue;
+        if (evictable++ == 0 || ps.plans[i].last_use < ps.plans[at].last_use) at = i;
+    }
+    if (evictable < kPrefillPlans || pl.captured) {
+        at = ps.plans.size();
+        ps.plans.emplace_back();
+    } else {
         // Kernels on any stream may still read the evicted table.
         G4_HIP(hipDeviceSynchronize());
         std::swap(pl.mem, ps.plans[at].mem);
         std::swap(pl.mem_bytes, ps.plans[at].mem_bytes);
         ps.plans[at].pos0 = -1;  // no shape's table until the new one is in
-    } else {
-        ps.plans.emplace_back();
     }
     PrefillPlan &slot = ps.plans[at];
     hipError_t e = hipSuccess;
@@ -1786,7 +1792,7 @@ int launch_prefill(g4_ctx *ctx, const PrefillArgs &a, hipStream_t stream) {
     const bool split = !ctx->prefill_exact && plane_bytes < (1ull << 31) && std::isfinite(a.scale) &&
                        std::fabs(a.scale) <= 4294967296.0f;
     const PrefillPlan *plp = nullptr;
-    int rc = plan_for(ctx, a, split, &plp);
+    int rc = plan_for(ctx, a, split, stream, &plp);
     if (rc != G4_OK) return rc;
     const PrefillPlan &pl = *plp;
     PrefillK p{};

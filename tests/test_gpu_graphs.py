@@ -84,6 +84,48 @@ def test_prefill_in_a_graph(ctx, d, window):
                      lambda i: [torch.randn(N, 8 * d, device="cuda"), torch.randn(N, d, device="cuda")])
 
 
+@pytest.mark.parametrize("d,window,pos0,N", [(512, 0, 0, 300), (256, 512, 700, 40), (512, 0, 4000, 17)])
+def test_prefill_graph_outlives_its_shapes_turn_in_the_table_cache(d, window, pos0, N):
+    """A context keeps the schedule tables of the last 128 prefill shapes; a
+    captured graph's table stays beyond that.  The graph replays between and
+    after eager calls of 160 other shapes."""
+    import g4hip
+    rng = np.random.default_rng(d + pos0)
+    q = dev(rng.standard_normal((N, 8 * d)).astype(np.float32))
+    K = dev(rng.standard_normal((pos0 + N, d)).astype(np.float32))
+    V = dev(rng.standard_normal((pos0 + N, d)).astype(np.float32))
+    out = torch.zeros(N * 8 * d, device="cuda")
+    other = torch.zeros(300 * 8 * d, device="cuda")
+    with g4hip.Context(0) as ctx:
+        big = torch.zeros(1024, 8 * 512, device="cuda")  # the largest workspace first: it does not grow later
+        ctx.attend_prefill(big, big, big, 0, 1024, 0, 8, 1, 512, torch.zeros_like(big))
+        deep = torch.zeros(8200, 512, device="cuda")
+        ctx.attend_prefill(big, deep, deep, 8000, 64, 0, 8, 1, 512, torch.zeros_like(big))
+
+        def run():
+            ctx.attend_prefill(q, K, V, pos0, N, window, 8, 1, d, out)
+
+        run()
+        ref = out.clone()
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            run()
+        for i in range(160):
+            n = 1 + i % min(N, pos0 + N - 1)
+            ctx.attend_prefill(q, K, V, i % (pos0 + N - n), n, 1 + i, 8, 1, d, other)
+            if i % 40 == 39:
+                out.fill_(float("nan"))
+                torch.cuda.synchronize()
+                g.replay()
+                torch.cuda.synchronize()
+                assert torch.equal(out, ref), f"after {i + 1} other shapes"
+        run()
+        torch.cuda.synchronize()
+        assert torch.equal(out, ref)
+        ctx.check_status()
+
+
 def test_prepare_and_decode_step_in_a_graph(ctx):
     """A global layer step: fused q/k/v preparation with the append into the
     cache, then the decode over the cache."""
