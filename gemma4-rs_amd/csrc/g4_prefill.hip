@@ -1631,18 +1631,29 @@ static std::vector<std::pair<int, int>> block_tile_ranges(int64_t pos0, int64_t 
 static int bins_for(int num_cus, int n_kv_heads) { return std::max(1, num_cus / std::max(1, n_kv_heads)); }
 
 // The schedule tables of a's shape: cached, or built and uploaded
-// (synchronously: graph capture needs an earlier call with the same shape).
+// (synchronously: graph capture needs an earlier call with the same shape,
+// in either form).
 static int plan_for(g4_ctx *ctx, const PrefillArgs &a, bool split, hipStream_t stream, const PrefillPlan **out) {
     PrefillPlans &ps = plans_of(ctx);
     ++ps.tick;
+    const bool recording = capturing(stream);
+    PrefillPlan *found = nullptr;
     for (auto &pl : ps.plans)
         if (pl.pos0 == a.pos0 && pl.N == a.N && pl.window == a.window && pl.head_dim == a.head_dim &&
-            pl.n_kv_heads == a.n_kv_heads && pl.split == split) {
-            pl.last_use = ps.tick;
-            pl.captured |= capturing(stream);
-            *out = &pl;
-            return G4_OK;
+            pl.n_kv_heads == a.n_kv_heads) {
+            // The forms differ in what a tile costs, not in what a table
+            // means: a capture, which can build none, takes the other form's.
+            if (pl.split == split)
+                found = &pl;
+            else if (recording && !found)
+                found = &pl;
         }
+    if (found) {
+        found->last_use = ps.tick;
+        found->captured |= recording;
+        *out = found;
+        return G4_OK;
+    }
     const std::vector<std::pair<int, int>> bt = block_tile_ranges(a.pos0, a.N, a.window);
     Bins bins;
     int slices = 1;
@@ -1677,7 +1688,7 @@ static int plan_for(g4_ctx *ctx, const PrefillArgs &a, bool split, hipStream_t s
     pl.n_blocks = (int)blocks.size();
     pl.n_slots = n_slots;
     pl.last_use = ps.tick;
-    pl.captured = capturing(stream);
+    pl.captured = recording;
     // One image of the tables, one copy.
     std::vector<PrefillBin> table(pl.n_bins);
     for (int b = 0; b < pl.n_bins; ++b) table[b] = {bin_start[b], bin_start[b + 1], {0, 0}, units[bin_start[b]]};

@@ -126,6 +126,47 @@ def test_prefill_graph_outlives_its_shapes_turn_in_the_table_cache(d, window, po
         ctx.check_status()
 
 
+@pytest.mark.parametrize("captured", [1, 0])
+@pytest.mark.parametrize("d,window,pos0,N", [(512, 0, 0, 300), (256, 512, 700, 40), (512, 0, 4000, 17)])
+def test_prefill_capture_in_the_other_form_than_the_warm_up(d, window, pos0, N, captured):
+    """One eager call makes a shape's capture possible in either product form:
+    nothing is allocated or copied then."""
+    import g4hip
+    from oracle import pyoracle as orc
+    rng = np.random.default_rng(d + pos0 + captured)
+    qn = rng.standard_normal((N, 8 * d), dtype=np.float32) * 0.3
+    Kn, Vn = (rng.standard_normal((pos0 + N, d), dtype=np.float32) for _ in range(2))
+    q, K, V = dev(qn), dev(Kn), dev(Vn)
+    out = torch.zeros(N * 8 * d, device="cuda")
+    ref, status = orc.attend_prefill(qn, Kn, Vn, pos0, window, 8, 1)
+    assert not status.any()
+    with g4hip.Context(0) as ctx:
+        def run():
+            ctx.attend_prefill(q, K, V, pos0, N, window, 8, 1, d, out)
+
+        big = torch.zeros(8200, 8 * 512, device="cuda")  # a workspace large enough for both forms
+        ctx.attend_prefill(big, big, big, 8000, 64, 0, 8, 1, 512, torch.zeros(64, 8 * 512, device="cuda"))
+        ctx.set_prefill_exact(1 - captured)
+        run()
+        torch.cuda.synchronize()
+        ctx.set_prefill_exact(captured)
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            run()
+        for _ in range(3):
+            out.fill_(float("nan"))
+            torch.cuda.synchronize()
+            g.replay()
+            torch.cuda.synchronize()
+            got = out.cpu().numpy().reshape(N, -1)
+            assert max(I.rel_err(got[i], ref[i]) for i in range(N)) <= 1e-4
+            run()  # the form's own table from here on
+            torch.cuda.synchronize()
+            got = out.cpu().numpy().reshape(N, -1)
+            assert max(I.rel_err(got[i], ref[i]) for i in range(N)) <= 1e-4
+        ctx.check_status()
+
+
 def test_prepare_and_decode_step_in_a_graph(ctx):
     """A global layer step: fused q/k/v preparation with the append into the
     cache, then the decode over the cache."""
