@@ -1,6 +1,7 @@
 // C ABI entry points: context, errors, attention calls, device KvCache, the
 // layer attention driver, the engine's policies and the ComputePort methods.
 
+#include <algorithm>
 #include <climits>
 #include <math.h>
 #include <new>
@@ -60,31 +61,39 @@ bool capturing(hipStream_t stream) {
     return st == hipStreamCaptureStatusActive;
 }
 
-int ensure_workspace(g4_ctx *ctx, size_t bytes, hipStream_t stream) {
-    (void)stream;
-    if (ctx->ws.bytes >= bytes) return G4_OK;
-    // Growth is rare (first use of a larger shape): drain all work that may
-    // still read the old buffer before replacing it.
-    G4_HIP(hipDeviceSynchronize());
-    if (ctx->ws.ptr) G4_HIP(hipFree(ctx->ws.ptr));
-    ctx->ws.ptr = nullptr;
-    ctx->ws.bytes = 0;
-    const size_t grown = bytes + bytes / 4;
-    G4_HIP(hipMalloc(&ctx->ws.ptr, grown));
-    ctx->ws.bytes = grown;
+// Grows w to `grown` bytes if it has fewer than `bytes`.  Growth is rare
+// (first use of a larger shape): drain all work that may still read the old
+// buffer before replacing it.  A graph that was captured over the old buffer
+// uses it at every replay, so such a buffer stays until the context goes.
+// Each is at least a quarter larger than the one before: together they hold
+// at most four times the current one's bytes.
+static int grow(g4_ctx *ctx, Workspace &w, size_t bytes, size_t grown, hipStream_t stream) {
+    if (w.bytes < bytes) {
+        G4_HIP(hipDeviceSynchronize());
+        if (w.ptr && w.captured)
+            ctx->outgrown.push_back(w.ptr);
+        else if (w.ptr)
+            G4_HIP(hipFree(w.ptr));
+        w = Workspace{};
+        G4_HIP(hipMalloc(&w.ptr, grown));
+        w.bytes = grown;
+    }
+    w.captured = w.captured || capturing(stream);
     return G4_OK;
 }
 
-int ensure_zero_rows(g4_ctx *ctx, int64_t n) {
-    if (ctx->zero_rows_len >= n) return G4_OK;
-    G4_HIP(hipDeviceSynchronize());
-    if (ctx->zero_rows) G4_HIP(hipFree(ctx->zero_rows));
-    ctx->zero_rows = nullptr;
-    ctx->zero_rows_len = 0;
-    const int64_t len = n < 1024 ? 1024 : n;
-    G4_HIP(hipMalloc(&ctx->zero_rows, len * sizeof(int64_t)));
-    G4_HIP(hipMemset(ctx->zero_rows, 0, len * sizeof(int64_t)));
-    ctx->zero_rows_len = len;
+int ensure_workspace(g4_ctx *ctx, size_t bytes, hipStream_t stream) {
+    return grow(ctx, ctx->ws, bytes, bytes + bytes / 4, stream);
+}
+
+int ensure_zero_rows(g4_ctx *ctx, int64_t n, hipStream_t stream) {
+    const size_t had = ctx->zero_rows.bytes, need = (size_t)n * sizeof(int64_t);
+    const int rc = grow(ctx, ctx->zero_rows, need, std::max(need + need / 4, (size_t)1024 * sizeof(int64_t)), stream);
+    if (rc != G4_OK || ctx->zero_rows.bytes == had) return rc;
+    const size_t bytes = ctx->zero_rows.bytes;
+    ctx->zero_rows.bytes = 0;  // until they are zero
+    G4_HIP(hipMemset(ctx->zero_rows.ptr, 0, bytes));
+    ctx->zero_rows.bytes = bytes;
     return G4_OK;
 }
 
@@ -193,7 +202,8 @@ int g4_release(g4_ctx *ctx) {
         G4_HIP(hipSetDevice(ctx->device));
         G4_HIP(hipDeviceSynchronize());
         if (ctx->ws.ptr) G4_HIP(hipFree(ctx->ws.ptr));
-        if (ctx->zero_rows) G4_HIP(hipFree(ctx->zero_rows));
+        if (ctx->zero_rows.ptr) G4_HIP(hipFree(ctx->zero_rows.ptr));
+        for (void *p : ctx->outgrown) G4_HIP(hipFree(p));
         g4::release_prefill_plan(ctx);
         if (ctx->status_dev) G4_HIP(hipFree(ctx->status_dev));
         delete ctx;

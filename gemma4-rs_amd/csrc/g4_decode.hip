@@ -1356,9 +1356,9 @@ int launch_decode(g4_ctx *ctx, const DecodeArgs &a, hipStream_t stream) {
     if (a.prefill_window >= 0) return launch_mode<kPrefill>(ctx, a, p, stream);
     if (a.kv_begin) {
         if (!p.seq_row0) {  // a zero row offset for every sequence
-            int rc = ensure_zero_rows(ctx, a.B);
+            int rc = ensure_zero_rows(ctx, a.B, stream);
             if (rc != G4_OK) return rc;
-            p.seq_row0 = ctx->zero_rows;
+            p.seq_row0 = (const int64_t *)ctx->zero_rows.ptr;
         }
         return launch_mode<kBatch>(ctx, a, p, stream);
     }

@@ -6,6 +6,7 @@
 #include <cstdint>
 #include <cstdio>
 #include <string>
+#include <vector>
 
 #include "../../include/g4attn.h"
 
@@ -30,9 +31,11 @@ enum : unsigned {
     kStatusRangeTooLong = 2u // a ragged range exceeded max_kv_len
 };
 
+// A device buffer that grows on demand.
 struct Workspace {
     void *ptr = nullptr;
     size_t bytes = 0;
+    bool captured = false;  // a graph holds its address
 };
 
 }  // namespace g4
@@ -44,8 +47,8 @@ struct g4_ctx {
     int64_t decode_chunk = 0;        // 0 = automatic
     int prefill_exact = 0;           // 1: prefill uses f32 MFMAs only (no split-f16 products)
     int num_cus = 256;
-    int64_t *zero_rows = nullptr;    // device zeros: default row offsets of a batch
-    int64_t zero_rows_len = 0;
+    g4::Workspace zero_rows;         // device zeros (int64): default row offsets of a batch
+    std::vector<void *> outgrown;    // buffers that grew while a graph held their address
     void *prefill_plan = nullptr;    // work-unit tables of the last prefill shapes
     void *scratch = nullptr;         // this device's static decode scratch (g4_attend_decode_noalloc)
     size_t scratch_bytes = 0;
@@ -61,7 +64,7 @@ bool capturing(hipStream_t stream);
 // must not be in flight on another stream when it grows).
 int ensure_workspace(g4_ctx *ctx, size_t bytes, hipStream_t stream);
 // Makes ctx->zero_rows hold at least n zero int64 values.
-int ensure_zero_rows(g4_ctx *ctx, int64_t n);
+int ensure_zero_rows(g4_ctx *ctx, int64_t n, hipStream_t stream);
 
 // Launchers implemented in the .hip files.
 struct DecodeArgs {

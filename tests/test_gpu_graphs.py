@@ -226,3 +226,59 @@ def test_fused_decode_step_in_a_graph(ctx):
     replay_and_check(ctx, run, [q, k, v], [out],
                      lambda i: [torch.randn(8 * d, device="cuda"), torch.randn(d, device="cuda"),
                                 torch.randn(d, device="cuda")])
+
+
+def _rows(rng, n, width):
+    return dev(rng.standard_normal((n, width), dtype=np.float32) * 0.3)
+
+
+@pytest.mark.parametrize("call", ["decode", "ragged", "ragged_row0", "stream", "prefill", "few_queries", "softcap"])
+def test_graphs_outlive_the_growth_of_the_workspace(call):
+    """A captured call keeps the context's buffers of its time; larger eager
+    calls grow them twice between replays."""
+    import g4hip
+    rng = np.random.default_rng(5)
+    d = 512
+    out = torch.zeros(64 * 8 * d, device="cuda")
+    with g4hip.Context(0) as ctx:
+        if call == "decode":
+            q, K, V, n = _rows(rng, 1, 8 * d), _rows(rng, 1000, d), _rows(rng, 1000, d), 8 * d
+            run = lambda: ctx.attend_decode(q, K, V, 0, 1000, 8, 1, d, out)
+        elif call in ("ragged", "ragged_row0", "stream"):
+            lens = np.array([5, 700, 64, 333], np.int64) * (30 if call == "stream" else 1)
+            longest, n = int(lens.max()), 4 * 8 * d
+            q, K, V = _rows(rng, 4, 8 * d), _rows(rng, longest, d), _rows(rng, longest, d)
+            begin, end, row0 = dev(lens * 0), dev(lens), dev(lens * 0) if call != "ragged_row0" else None
+            run = lambda: ctx.attend_decode_batch(q, K, V, row0, begin, end, longest, 8, 1, d, out)
+        elif call == "softcap":
+            x = _rows(rng, 1, 1536)
+            w = dev(np.tile(I.q8_0_bytes(rng.uniform(-1, 1, 1000 * 1536).astype(np.float32)), 90))
+            n = 90000
+            run = lambda: ctx.logits_q8_0(w, 90000, 1536, x, 30.0, out)
+        else:
+            pos0, N = (0, 60) if call == "prefill" else (600, 9)
+            q, K, V, n = _rows(rng, N, 8 * d), _rows(rng, pos0 + N, d), _rows(rng, pos0 + N, d), N * 8 * d
+            run = lambda: ctx.attend_prefill(q, K, V, pos0, N, 0, 8, 1, d, out)
+        run()
+        ref = out.clone()
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            run()
+        big = _rows(rng, 20000, d)
+        bigq, bigout = _rows(rng, 64, 8 * d), torch.zeros(64 * 8 * d, device="cuda")
+        for rows, B in ((8000, 1500), (20000, 3000)):
+            ctx.attend_prefill(bigq, big, big, rows - 64, 64, 0, 8, 1, d, bigout)
+            ones = torch.ones(B, dtype=torch.int64, device="cuda")  # a batch that needs more row offsets
+            wide = torch.zeros(B, 8 * 256, device="cuda")
+            ctx.attend_decode_batch(wide, big, big, None, ones * 0, ones, 1, 8, 1, 256, torch.zeros_like(wide))
+            for _ in range(2):
+                out.fill_(float("nan"))
+                torch.cuda.synchronize()
+                g.replay()
+                torch.cuda.synchronize()
+                assert torch.equal(out[:n], ref[:n])
+        run()
+        torch.cuda.synchronize()
+        assert torch.equal(out[:n], ref[:n])
+        ctx.check_status()
