@@ -129,6 +129,14 @@ struct PrefillUnit {
     int slot;    // partial slot, or -1 when the block has a single unit
 };
 
+// Workgroup z's share of a unit's tiles, with its partial slot, where
+// `slices` workgroups share each unit (the schedule leaves each at least one
+// tile).
+__host__ __device__ inline PrefillUnit slice_of(const PrefillUnit &u, int z, int slices) {
+    const int n = u.t_hi - u.t_lo;
+    return {u.block, u.t_lo + n * z / slices, u.t_lo + n * (z + 1) / slices, u.slot * slices + z};
+}
+
 // A workgroup's units [first, end) of the table, and the first of them (one
 // load tells a workgroup where it starts).
 struct PrefillBin {
@@ -1116,12 +1124,7 @@ __global__ __launch_bounds__(PrefillShape<D>::THREADS, 1) void prefill_kernel(Pr
             __syncthreads();
             u = p.units[i];
         }
-        if (p.slices > 1) {  // this workgroup's share (the host leaves each at least one tile)
-            const int n = u.t_hi - u.t_lo, z = slice, lo = u.t_lo;
-            u.t_lo = lo + n * z / p.slices;
-            u.t_hi = lo + n * (z + 1) / p.slices;
-            u.slot = u.slot * p.slices + z;
-        }
+        if (p.slices > 1) u = slice_of(u, slice, p.slices);
         if (p.planes != nullptr && prefill_unit<D, true>(p, u, kvh, L)) continue;
         if (p.planes != nullptr) __syncthreads();  // the declined split form's tiles have landed
         prefill_unit<D, false>(p, u, kvh, L);
@@ -1571,10 +1574,20 @@ static int build_schedule(const BlockTiles &bt, int n_bins, const ScheduleCost &
     return 0;
 }
 
-// The unit table, workgroup ranges and block table of a schedule; checks
-// that every block's pieces tile its range exactly.
-static int schedule_tables(const std::vector<std::pair<int, int>> &bt, Bins &bins, std::vector<PrefillUnit> &units,
-                           std::vector<int> &bin_start, std::vector<PrefillBlockInfo> &blocks, int &n_slots) {
+// The unit table, workgroup ranges and block table of a schedule.
+struct Schedule {
+    std::vector<PrefillUnit> units;
+    std::vector<int> bin_start;
+    std::vector<PrefillBlockInfo> blocks;
+    int n_slots = 0;
+    int slices = 1;
+};
+
+// Fills in a schedule's tables from its bins; checks that every block's
+// pieces tile its range exactly.
+static int schedule_tables(const BlockTiles &bt, Bins &bins, Schedule &out) {
+    auto &[units, bin_start, blocks, n_slots, slices] = out;
+    (void)slices;
     const int n_blocks = (int)bt.size();
     bins.erase(std::remove_if(bins.begin(), bins.end(), [](const std::vector<Piece> &x) { return x.empty(); }),
                bins.end());
@@ -1614,6 +1627,19 @@ static int schedule_tables(const std::vector<std::pair<int, int>> &bt, Bins &bin
     return G4_OK;
 }
 
+// Slots and partial counts where several workgroups share each unit: every
+// unit leaves a partial per slice, unit slot s those at s * slices onwards.
+static void number_slices(Schedule &s) {
+    if (s.slices == 1) return;
+    for (PrefillUnit &u : s.units)
+        if (u.slot < 0) {
+            u.slot = s.n_slots++;
+            s.blocks[u.block] = {u.slot, 1};
+        }
+    for (PrefillBlockInfo &b : s.blocks) b = {b.first_slot * s.slices, b.n_units * s.slices};
+    s.n_slots *= s.slices;
+}
+
 // [t_lo, t_hi) tiles of each position block of a prefill shape.
 static std::vector<std::pair<int, int>> block_tile_ranges(int64_t pos0, int64_t N, int64_t window) {
     const int n_blocks = (int)((N + kPosPerBlock - 1) / kPosPerBlock);
@@ -1628,7 +1654,16 @@ static std::vector<std::pair<int, int>> block_tile_ranges(int64_t pos0, int64_t 
     return bt;
 }
 
-static int bins_for(int num_cus, int n_kv_heads) { return std::max(1, num_cus / std::max(1, n_kv_heads)); }
+// The schedule of a prefill shape, its slots not yet numbered by slice.
+static int make_schedule(int64_t pos0, int64_t N, int64_t window, int head_dim, int n_kv_heads, int num_cus, bool split,
+                         Schedule &out) {
+    const BlockTiles bt = block_tile_ranges(pos0, N, window);
+    const int n_bins = std::max(1, num_cus / std::max(1, n_kv_heads));
+    Bins bins;
+    if (build_schedule(bt, n_bins, cost_of(head_dim, split), bins, &out.slices) != 0)
+        return set_error(G4_ERR_COMPUTE, "prefill key range too long for one call");
+    return schedule_tables(bt, bins, out);
+}
 
 // The schedule tables of a's shape: cached, or built and uploaded
 // (synchronously: graph capture needs an earlier call with the same shape,
@@ -1654,27 +1689,12 @@ static int plan_for(g4_ctx *ctx, const PrefillArgs &a, bool split, hipStream_t s
         *out = found;
         return G4_OK;
     }
-    const std::vector<std::pair<int, int>> bt = block_tile_ranges(a.pos0, a.N, a.window);
-    Bins bins;
-    int slices = 1;
-    if (build_schedule(bt, bins_for(ctx->num_cus, a.n_kv_heads), cost_of(a.head_dim, split), bins, &slices) != 0)
-        return set_error(G4_ERR_COMPUTE, "prefill key range too long for one call");
-    std::vector<PrefillUnit> units;
-    std::vector<int> bin_start;
-    std::vector<PrefillBlockInfo> blocks;
-    int n_slots = 0;
-    int rc = schedule_tables(bt, bins, units, bin_start, blocks, n_slots);
+    Schedule sched;
+    const int rc = make_schedule(a.pos0, a.N, a.window, a.head_dim, a.n_kv_heads, ctx->num_cus, split, sched);
     if (rc != G4_OK) return rc;
+    number_slices(sched);
+    const auto &[units, bin_start, blocks, n_slots, slices] = sched;
     PrefillPlan pl;
-    if (slices > 1) {  // every unit leaves a partial per slice
-        for (PrefillUnit &u : units)
-            if (u.slot < 0) {
-                u.slot = n_slots++;
-                blocks[u.block] = {u.slot, 1};
-            }
-        for (PrefillBlockInfo &b : blocks) b = {b.first_slot * slices, b.n_units * slices};
-        n_slots *= slices;
-    }
     for (const PrefillBlockInfo &b : blocks) pl.max_parts = std::max(pl.max_parts, b.n_units);
     pl.slices = slices;
     pl.split = split;
@@ -1737,31 +1757,27 @@ static int plan_for(g4_ctx *ctx, const PrefillArgs &a, bool split, hipStream_t s
 }
 
 int describe_prefill_schedule(int64_t pos0, int64_t N, int64_t window, int head_dim, int n_kv_heads, int num_cus,
-                              int32_t *units4, int64_t units_cap, int32_t *bin_start_out, int64_t bins_cap,
-                              int32_t *counts) {
-    const std::vector<std::pair<int, int>> bt = block_tile_ranges(pos0, N, window);
-    Bins bins;
-    int slices = 1;
-    if (build_schedule(bt, bins_for(num_cus, n_kv_heads), cost_of(head_dim, true), bins, &slices) != 0)
-        return set_error(G4_ERR_COMPUTE, "prefill key range too long for one call");
-    std::vector<PrefillUnit> units;
-    std::vector<int> bin_start;
-    std::vector<PrefillBlockInfo> blocks;
-    int n_slots = 0;
-    int rc = schedule_tables(bt, bins, units, bin_start, blocks, n_slots);
+                              bool split, bool launched, int32_t *units4, int64_t units_cap, int32_t *bin_start_out,
+                              int64_t bins_cap, int32_t *counts) {
+    Schedule s;
+    const int rc = make_schedule(pos0, N, window, head_dim, n_kv_heads, num_cus, split, s);
     if (rc != G4_OK) return rc;
-    counts[0] = (int32_t)units.size();
-    counts[1] = (int32_t)bin_start.size() - 1;
-    counts[2] = n_slots;
-    if ((int64_t)units.size() > units_cap || (int64_t)bin_start.size() > bins_cap)
+    const int slices = launched ? s.slices : 1, n_units = (int)s.units.size(), n_bins = (int)s.bin_start.size() - 1;
+    if (launched) number_slices(s);
+    counts[0] = n_units * slices;
+    counts[1] = n_bins * slices;
+    counts[2] = s.n_slots;
+    if (counts[0] > units_cap || counts[1] + 1 > bins_cap)
         return set_error(G4_ERR_MSG, "prefill schedule: output arrays too small");
-    for (size_t i = 0; i < units.size(); ++i) {
-        units4[4 * i] = units[i].block;
-        units4[4 * i + 1] = units[i].t_lo;
-        units4[4 * i + 2] = units[i].t_hi;
-        units4[4 * i + 3] = units[i].slot;
+    for (int z = 0; z < slices; ++z) {
+        for (int i = 0; i < n_units; ++i) {
+            const PrefillUnit u = slices > 1 ? slice_of(s.units[i], z, slices) : s.units[i];
+            const int32_t row[4] = {u.block, u.t_lo, u.t_hi, u.slot};
+            memcpy(units4 + 4 * ((size_t)z * n_units + i), row, sizeof row);
+        }
+        for (int b = 0; b < n_bins; ++b) bin_start_out[z * n_bins + b] = z * n_units + s.bin_start[b];
     }
-    for (size_t i = 0; i < bin_start.size(); ++i) bin_start_out[i] = bin_start[i];
+    bin_start_out[counts[1]] = counts[0];
     return G4_OK;
 }
 

@@ -246,6 +246,39 @@ impl HipPort {
     }
 }
 
+/// The work schedule that `attend_prefill` launches for a shape, in split-f16
+/// or (`exact`) f32 products: units of `[block, first tile, end tile, partial
+/// slot or -1]`, and each workgroup's first unit, the number of units last.
+pub fn prefill_launch_schedule(
+    pos0: usize,
+    n: usize,
+    window: usize,
+    head_dim: usize,
+    n_kv_heads: usize,
+    num_cus: usize,
+    exact: bool,
+) -> Result<(Vec<[i32; 4]>, Vec<i32>), EngError> {
+    let (p0, nn, w) = (len_i64(pos0)?, len_i64(n)?, len_i64(window)?);
+    let (hd, nkv) = (to_c_int(head_dim, "head_dim")?, to_c_int(n_kv_heads, "n_kv_heads")?);
+    let (cus, ex) = (to_c_int(num_cus, "num_cus")?, exact as c_int);
+    let mut counts = [0i32; 3];
+    let pc = counts.as_mut_ptr();
+    let run = |units: &mut [[i32; 4]], bins: &mut [i32]| -> Result<c_int, EngError> {
+        let (uc, bc) = (len_i64(units.len())?, len_i64(bins.len())?);
+        let (pu, pb) = (units.as_mut_ptr().cast::<i32>(), bins.as_mut_ptr());
+        // SAFETY: the arrays hold the capacities given, counts three values.
+        Ok(unsafe { ffi::g4_prefill_launch_schedule(p0, nn, w, hd, nkv, cus, ex, pu, uc, pb, bc, pc) })
+    };
+    let code = run(&mut [[0; 4]; 1], &mut [0; 1])?; // the sizes
+    if code != ffi::G4_ERR_MSG {
+        check(code)?;
+    }
+    let mut units = vec![[0i32; 4]; counts[0] as usize];
+    let mut bins = vec![0i32; counts[1] as usize + 1];
+    check(run(&mut units, &mut bins)?)?;
+    Ok((units, bins))
+}
+
 /// `layer_attention_kind` (idea/mod.rs:148-156): true on global layers.
 pub fn layer_is_global(n_layers: usize, layer: usize) -> Result<bool, EngError> {
     let (n, l) = (to_c_int(n_layers, "n_layers")?, to_c_int(layer, "layer")?);

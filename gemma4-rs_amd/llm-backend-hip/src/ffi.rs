@@ -164,6 +164,20 @@ extern "C" {
         bins_cap: i64,
         counts: *mut i32,
     ) -> c_int;
+    pub fn g4_prefill_launch_schedule(
+        pos0: i64,
+        n: i64,
+        window: i64,
+        head_dim: c_int,
+        n_kv_heads: c_int,
+        num_cus: c_int,
+        exact: c_int,
+        units: *mut i32,
+        units_cap: i64,
+        bin_start: *mut i32,
+        bins_cap: i64,
+        counts: *mut i32,
+    ) -> c_int;
     pub fn g4_rms_norm_rows(
         ctx: *mut G4Ctx,
         x_dev: *const f32,

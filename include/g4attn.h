@@ -156,19 +156,30 @@ int g4_attend_prefill(g4_ctx *ctx, const float *q_dev, const float *k_cache_dev,
 
 /* Work schedule of g4_attend_prefill's MFMA path (head_dim 256 or 512,
  * 8 query heads per KV head) on a GPU with num_cus compute units: position
- * blocks of 8 queries are cut into units of 16-key tiles, and workgroup w
- * (of n_bins per KV head) runs units bin_start[w] .. bin_start[w+1]-1 in
- * turn.  units (host) gets 4 int32 per unit: {block, first tile, end tile,
- * partial slot or -1 for a block computed by one unit}; bin_start (host)
- * n_bins+1 entries; counts (host) {n_units, n_bins, n_slots}.  Where the bins
- * do not fill the GPU, a unit's tiles are shared out further, over several
- * workgroups that each leave a partial (not listed here).  Host only,
- * no device work; counts are filled even when the arrays are too small
- * (then G4_ERR_MSG).  No counterpart in the reference, whose prompt runs
- * token at a time (crates/llm-gemma4/src/impl_/generate.rs:37-41). */
+ * blocks of 8 queries are cut into at most 8 units of 16-key tiles, and
+ * workgroup w (of n_bins per KV head) runs units bin_start[w] ..
+ * bin_start[w+1]-1 in turn.  units (host) gets 4 int32 per unit: {block,
+ * first tile, end tile, partial slot or -1 for a block computed by one
+ * unit}; bin_start (host) n_bins+1 entries; counts (host) {n_units, n_bins,
+ * n_slots}.  For the default (split-f16) products, and before the units are
+ * shared out where the bins do not fill the GPU: g4_prefill_launch_schedule
+ * gives what a call launches.  Host only, no device work; counts are filled
+ * even when the arrays are too small (then G4_ERR_MSG).  No counterpart in
+ * the reference, whose prompt runs token at a time
+ * (crates/llm-gemma4/src/impl_/generate.rs:37-41). */
 int g4_prefill_schedule(int64_t pos0, int64_t N, int64_t window, int head_dim, int n_kv_heads, int num_cus,
                         int32_t *units, int64_t units_cap, int32_t *bin_start, int64_t bins_cap,
                         int32_t *counts);
+
+/* The same as a call launches it, in the default products (exact 0) or in
+ * f32 MFMAs (exact 1, g4_set_prefill_exact), whose tiles cost differently.
+ * Where the units of g4_prefill_schedule do not fill the GPU, several
+ * workgroups share each unit's tiles and leave a partial each: they are
+ * listed as workgroups and units of their own, so a block can have more than
+ * 8 units. */
+int g4_prefill_launch_schedule(int64_t pos0, int64_t N, int64_t window, int head_dim, int n_kv_heads, int num_cus,
+                               int exact, int32_t *units, int64_t units_cap, int32_t *bin_start,
+                               int64_t bins_cap, int32_t *counts);
 
 /* ----------------------------------------- attention input preparation */
 /* rms_norm (crates/llm-backend-cpu/src/ops.rs:45-56) applied to each of

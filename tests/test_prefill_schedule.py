@@ -112,3 +112,58 @@ def test_schedule_rejects_bad_shapes():
             g4hip.prefill_schedule(*args)
     with pytest.raises(g4hip.EngError):
         g4hip.prefill_schedule(0, 16, 0, 512, 0, 256)
+
+
+FEW = [  # few queries deep in a context: units shared over slices
+    (16384, 8, 0, 512, 1), (4000, 64, 0, 512, 1), (2500, 17, 0, 512, 2), (300, 1, 0, 512, 1), (9000, 9, 0, 256, 4),
+    (5000, 25, 512, 256, 1), (7000, 40, 4096, 256, 2), (100000, 3, 0, 512, 1),
+]
+
+
+@pytest.mark.parametrize("exact", [0, 1])
+@pytest.mark.parametrize("pos0,N,window,d,n_kv", SHAPES + _drawn_shapes() + FEW)
+def test_launched_schedule(pos0, N, window, d, n_kv, exact):
+    """What a call launches, in both product forms: every attended tile of a
+    block once, workgroups for at most every CU, and each block's partials a
+    run of slots in key order.  Where the units leave CUs idle they are shared
+    out; no share is shorter than 4 tiles."""
+    units, bins = g4hip.prefill_launch_schedule(pos0, N, window, d, n_kv, 256, exact)
+    need = needed_tiles(pos0, N, window)
+    pieces = [[] for _ in need]
+    for b, lo, hi, slot in units.tolist():
+        assert 0 <= b < len(need) and lo < hi
+        pieces[b].append((lo, hi, slot))
+    used = []
+    for b, tiles in enumerate(need):
+        p = sorted(pieces[b])
+        assert p[0][0] == min(tiles) and p[-1][1] == max(tiles) + 1 and len(tiles) == max(tiles) + 1 - min(tiles)
+        assert all(x[1] == y[0] for x, y in zip(p, p[1:])), b
+        if len(p) == 1:
+            assert p[0][2] == -1
+            continue
+        assert [x[2] for x in p] == list(range(p[0][2], p[0][2] + len(p))), b
+        used += [x[2] for x in p]
+        if len(p) > 8:
+            assert min(hi - lo for lo, hi, _ in p) >= 4
+    assert sorted(used) == list(range(len(used)))
+    assert bins[0] == 0 and bins[-1] == len(units) and np.all(np.diff(bins) >= 1)
+    assert len(bins) - 1 <= 256 // n_kv
+
+
+@pytest.mark.parametrize("exact", [0, 1])
+def test_few_queries_fill_the_gpu(exact):
+    """8 queries over 16K keys: one block, more pieces than a block has units."""
+    units, bins = g4hip.prefill_launch_schedule(16384, 8, 0, 512, 1, 256, exact)
+    assert len(units) == len(bins) - 1 > 64
+    assert len(g4hip.prefill_schedule(16384, 8, 0, 512, 1, 256)[0]) <= 8  # before sharing
+
+
+def test_launched_schedule_depends_on_the_form():
+    """A unit costs 7 tiles in split products at d=512 and 1.9 in f32 ones."""
+    a, _ = g4hip.prefill_launch_schedule(0, 777, 0, 512, 1, 256, 0)
+    b, _ = g4hip.prefill_launch_schedule(0, 777, 0, 512, 1, 256, 1)
+    assert not np.array_equal(a, b)
+    with pytest.raises(g4hip.EngError):
+        g4hip.prefill_launch_schedule(0, 16, 0, 512, 1, 256, 2)
+    with pytest.raises(g4hip.EngError):
+        g4hip.prefill_launch_schedule(0, 16, 0, 128, 1, 256, 0)
