@@ -138,3 +138,37 @@ def test_few_queries_deep_in_a_context(ctx, d, window, pos0, N, exact):
     ref, status = orc.attend_prefill(q, K, V, pos0, window, 8, 1)
     assert not status.any()
     assert max(I.rel_err(got[i], ref[i]) for i in range(N)) <= TOL
+
+
+@pytest.mark.parametrize("far", [False, True])
+@pytest.mark.parametrize("d,window,pos0,N", [(512, 0, 4000, 64), (512, 0, 2500, 17), (256, 512, 5000, 25),
+                                             (256, 0, 9000, 9)])
+def test_few_queries_of_two_kv_heads_deep_in_a_context(ctx, d, window, pos0, N, far):
+    """The same with 2 KV heads, whose partials lie in turn.  far: the second
+    head holds one value beyond f16's range in K and one in V, so the pieces
+    that read them run in f32 among split-f16 ones."""
+    import g4hip
+    print(f"[case] few queries, 2 KV heads d={d} W={window} pos0={pos0} N={N} far={far}", flush=True)
+    units = [f(pos0, N, window, d, 2, 256)[0] for f in (g4hip.prefill_schedule, g4hip.prefill_launch_schedule)]
+    assert len(units[1]) > len(units[0])  # shared out over slices
+    q, K, V = (np.concatenate(x, axis=1) for x in zip(*(case(pos0 + N + s, pos0 + N, d, pos0) for s in (0, 50))))
+    if far:
+        q.reshape(N, 16, d)[:, 8:, 3] = 0.0
+        K[pos0 - 200, d + 3] = 1e5  # meets q's zeros
+        V[pos0 - 100, d + 7] = -1e5
+    out = torch.zeros(N * 16 * d, device="cuda")
+    ctx.attend_prefill(dev(q), dev(K), dev(V), pos0, N, window, 16, 2, d, out)
+    ctx.check_status()
+    got = out.cpu().numpy().reshape(N, -1)
+    ref, status = orc.attend_prefill(q, K, V, pos0, window, 16, 2)
+    assert not status.any()
+    assert max(I.rel_err(got[i], ref[i]) for i in range(N)) <= TOL
+    ctx.set_prefill_exact(1)
+    try:
+        ctx.attend_prefill(dev(q), dev(K), dev(V), pos0, N, window, 16, 2, d, out)
+    finally:
+        ctx.set_prefill_exact(0)
+    exact = out.cpu().numpy().reshape(N, 2, -1)
+    assert max(I.rel_err(exact[i].ravel(), ref[i]) for i in range(N)) <= TOL
+    for head in (0, 1):  # split pieces ran in both heads
+        assert not np.array_equal(got.reshape(N, 2, -1)[:, head], exact[:, head])
