@@ -1198,6 +1198,17 @@ void launch_merge(const DecodeK &p, int64_t n, int group, int n_kv_heads, int B,
                            stream, p);
 }
 
+// Whether a ragged batch of short contexts (units: sequences times KV heads)
+// keeps each in one split.  Once its splits fill half the chip, or its
+// sequences a third of it, another round of workgroups and the merge cost more
+// than a split's few tiles in a row.  Measured (us, whole / splits of 16 / 32):
+// 48 x 48 keys d=512 11.4 / 12.6 / 14.0, 32 x 48 11.1 / 10.7 / 12.4; 150 x 40
+// d=256 8.1 / 16.0 / 18, d=512 11.7 / 27 / 31; 100 x 96 d=512 16 / 27 / 27; 100
+// x 128 21 / 31 / 28, 64 x 128 19 / 21 / 18.
+bool whole_sequences(int64_t units, int64_t max_len, int64_t num_cus) {
+    return (max_len <= 64 && 2 * units * ((max_len + 15) / 16) > num_cus) || (max_len <= 128 && 3 * units > num_cus);
+}
+
 template <int MODE>
 int launch_mode(g4_ctx *ctx, const DecodeArgs &a, DecodeK p, hipStream_t stream,
                 const LayerPrepArgs *lp = nullptr) {
@@ -1234,7 +1245,10 @@ int launch_mode(g4_ctx *ctx, const DecodeArgs &a, DecodeK p, hipStream_t stream,
     // 16 / 32 / 64 keys): 8 x 512 keys d=256 7.5 / 8.6 / 10.8; 16 x 512 11.3 /
     // 10.2 / 11.6; 32 x 512 17.5 / 15.3 / 13.3; d=512, 8 of up to 579 keys 9.7
     // / 11.1 / 15.6; 5 of up to 1868 14.7 / 13.3 / 16.4; 26 of up to 636 19.7
-    // / 20.0 / 18.5.  Queries of a prompt: about eight per CU, at least 64
+    // / 20.0 / 18.5.  The bound says little of the lengths: 8 of up to 4000 keys
+    // (d=512) in splits of 64 / 96 / 128 take 36.4 / 37.9 / 30.5 all full, 28.7 /
+    // 21.2 / 24.9 evenly drawn, 15.9 / 18.2 / 21.7 one full and seven of 24
+    // keys.  Queries of a prompt: about eight per CU, at least 64
     // keys.  Contexts of up to two tiles run as one split (no merge); longer
     // ones split even when short: 64 keys took 6.8 us as one workgroup,
     // 5.7 us as four one-tile splits and the merge.
@@ -1247,7 +1261,7 @@ int launch_mode(g4_ctx *ctx, const DecodeArgs &a, DecodeK p, hipStream_t stream,
         if (MODE == kBatch) chunk = chunk <= 24 ? 16 : (chunk + 16) / 32 * 32;
         const int64_t floor_keys = MODE == kPrefill ? 64 : 16;
         if (chunk < floor_keys) chunk = floor_keys;
-        if (max_len <= 32) chunk = max_len;
+        if (max_len <= 32 || (MODE == kBatch && whole_sequences(units, max_len, ctx->num_cus))) chunk = max_len;
     }
     const int64_t min_chunk = (max_len + kMaxSplits - 1) / kMaxSplits;
     if (chunk < min_chunk) chunk = min_chunk;

@@ -218,3 +218,26 @@ def test_generic_prefill_after_non_finite_softmax_sums(ctx, chunk, pos0, N):
     got = out.cpu().numpy().reshape(N, -1)
     for i in range(N):
         assert I.rel_err(got[i], orc.attend(q[i], K[:pos0 + i + 1], V[:pos0 + i + 1], heads, 1)) <= TOL, i
+
+
+@pytest.mark.parametrize("d", [256, 512])
+@pytest.mark.parametrize("B,bound", [(32, 33), (32, 64), (33, 64), (43, 48), (85, 128), (86, 65), (86, 96), (86, 128),
+                                     (86, 129), (150, 40), (255, 128)])
+def test_ragged_short_contexts(ctx, d, B, bound):
+    """Batches on both sides of the line where each short context stays one
+    split, lengths from 1 to the bound."""
+    rng = np.random.default_rng(B * bound + d)
+    lens = rng.integers(1, bound + 1, B)
+    lens[:3] = 1, bound, (bound + 1) // 2
+    row0 = np.concatenate([[0], np.cumsum(lens)[:-1]]).astype(np.int64)
+    K = rng.standard_normal((int(lens.sum()), d), dtype=np.float32) * 0.1
+    V = rng.standard_normal((int(lens.sum()), d), dtype=np.float32)
+    q = rng.standard_normal((B, 8 * d), dtype=np.float32)
+    out = torch.full((B * 8 * d,), float("nan"), device="cuda")
+    ctx.attend_decode_batch(dev(q), dev(K), dev(V), dev(row0), dev(np.zeros(B, np.int64)), dev(lens.astype(np.int64)),
+                            bound, 8, 1, d, out)
+    ctx.check_status()
+    got = out.cpu().numpy().reshape(B, -1)
+    for s in range(B):
+        rows = slice(row0[s], row0[s] + lens[s])
+        assert I.rel_err(got[s], orc.attend(q[s], K[rows], V[rows], 8, 1)) <= TOL, s
