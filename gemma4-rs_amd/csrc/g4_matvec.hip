@@ -754,6 +754,30 @@ int launch_q8_once(g4_ctx *ctx, const MatvecArgs &a, hipStream_t stream, bool *d
     return G4_OK;
 }
 
+// Whether one lane per row is faster than matvec_q8_0_once_kernel, whose
+// wavefronts take a lane per block: where rows are so short that most lanes
+// idle and so many that the workgroups run in rounds, or so long that a CU's
+// LDS holds only a few.  Measured (us, lane per row / at once; the activation
+// quantized by a launch of its own in the first):
+//   int8 96 columns: 16,384 rows 6.2 / 5.8, 25,000 6.0 / 6.8, 100,000 7.1 / 13.5,
+//     262,144 9.8 / 29.9; 224: 32,768 8 / 7, 50,000 8 / 9; 256: 50,000 8 / 9,
+//     180,000 20 / 20; 16,384: 32,768 464 / 414, 40,000 467 / 503
+//   f32 512: 25,000 11.9 / 11.9, 65,536 14 / 23; 640: 32,768 13 / 14; 768: 50,000
+//     18 / 18, 100,000 31 / 28; 8192: 32,768 231 / 198, 50,000 243 / 304
+//   f64 256: 8192 10 / 9, 16,384 10 / 12, 262,144 14 / 84; 512: 32,768 13 / 16; 800:
+//     50,000 27 / 25, 131,072 40 / 52; 1024: 180,000 69 / 71, 262,144 115 / 101;
+//     4096: 32,768 116 / 93, 50,000 118 / 138
+template <int DOT, int NM>
+bool q8_lane_per_row(int64_t rows, int64_t nb, int64_t num_cus) {
+    const int64_t per_cu = rows / num_cus;
+    if (DOT == kInt8) {
+        if (nb > 256) return nb * rows > (NM == 2 ? 3LL << 23 : 1LL << 24);
+        return nb < 8 && per_cu >= 20 * std::max<int64_t>(nb, 4);
+    }
+    if (nb >= (DOT == kF32 ? 256 : 128)) return per_cu >= 160;
+    return nb <= (DOT == kF32 ? 20 : 28) && per_cu >= 8 * std::max<int64_t>(nb, DOT == kF32 ? 10 : 8);
+}
+
 template <int EPI>
 int launch_q8(g4_ctx *ctx, MatvecArgs a, hipStream_t stream) {
     constexpr int NM = EPI >= kGeglu ? 2 : 1;
@@ -773,7 +797,11 @@ int launch_q8(g4_ctx *ctx, MatvecArgs a, hipStream_t stream) {
     // 72.1.
     const bool large = staged && a.rows >= rb_max * 8 * num_cus &&
                        a.rows * nb * kQ8Bytes * NM > (512LL << 10) * num_cus;
-    if (!large) {
+    // The other two kernels read a quantized activation; a graph capture that
+    // finds no workspace for one can allocate none, and takes this one.
+    const size_t sbytes = ((size_t)nb * sizeof(float) + 255) / 256 * 256;
+    if (!(large || q8_lane_per_row<kInt8, NM>(a.rows, nb, num_cus)) ||
+        (!a.xs && ctx->ws.bytes < sbytes + (size_t)a.cols && capturing(stream))) {
         bool done = false;
         const int rc = launch_q8_once<EPI, kInt8>(ctx, a, stream, &done);
         if (rc != G4_OK || done) return rc;
@@ -781,7 +809,6 @@ int launch_q8(g4_ctx *ctx, MatvecArgs a, hipStream_t stream) {
     if (!a.xs) {
         // An f32 activation for a kernel that reads a quantized one:
         // quantize_q8_0 into the context's workspace first.
-        const size_t sbytes = ((size_t)nb * sizeof(float) + 255) / 256 * 256;
         const int rc = ensure_workspace(ctx, sbytes + (size_t)a.cols, stream);
         if (rc != G4_OK) return rc;
         a.xs = (const float *)ctx->ws.ptr;
@@ -812,9 +839,11 @@ int launch_q8(g4_ctx *ctx, MatvecArgs a, hipStream_t stream) {
 
 template <int DOT>
 int launch_q8_f32(g4_ctx *ctx, const MatvecArgs &a, hipStream_t stream) {
-    bool done = false;
-    const int rc = launch_q8_once<kPlain, DOT>(ctx, a, stream, &done);
-    if (rc != G4_OK || done) return rc;
+    if (!q8_lane_per_row<DOT, 1>(a.rows, a.cols / kQ8Values, ctx->num_cus)) {
+        bool done = false;
+        const int rc = launch_q8_once<kPlain, DOT>(ctx, a, stream, &done);
+        if (rc != G4_OK || done) return rc;
+    }
     hipLaunchKernelGGL(matvec_q8_0_f32_kernel<DOT == kF64>, dim3((unsigned)((a.rows + 255) / 256)), dim3(256), 0,
                        stream, a.w, a.rows, (int)(a.cols / kQ8Values), a.x, a.out);
     G4_HIP(hipGetLastError());

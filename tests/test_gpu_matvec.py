@@ -223,11 +223,11 @@ def test_fused_quantization_entries_equal_the_two_step_calls(ctx, rows, cols):
 
 
 @pytest.mark.parametrize("rows,cols", [(1, 32), (2, 64), (255, 96), (257, 1568), (2047, 160), (2049, 224), (4097, 544),
-                                       (9, 30016), (33000, 64)])
+                                       (9, 30016), (33000, 64), (20479, 128), (20480, 128), (35840, 224), (70000, 32)])
 @pytest.mark.parametrize("shift", [0, 2, 4])
 def test_q8_0_matvecs_at_the_tiles_edges(ctx, rows, cols, shift):
-    """Row counts around the wavefronts' shares, column counts whose rows
-    start anywhere (34-byte blocks, odd block counts), rows too long for one
+    """Row counts around the wavefronts' shares and around where short rows
+    go to a lane each, column counts whose rows start anywhere (34-byte blocks, odd block counts), rows too long for one
     workgroup per CU, and matrices 2 and 4 bytes off a 16-byte boundary: the
     quantized, the fused and both f32-activation forms, bit for bit."""
     print(f"[case] q8_0 {rows}x{cols} shift {shift}", flush=True)
