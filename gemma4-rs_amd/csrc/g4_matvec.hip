@@ -794,9 +794,11 @@ int launch_q8(g4_ctx *ctx, MatvecArgs a, hipStream_t stream) {
     // of its own, pays from some 128 MB on: 33,017 x 1024 (36 MB) 13.3 us
     // against 11.0 at once, 84,752 x 768 (69 MB) 20.4 against 17.2, 131,072 x
     // 1280 (178 MB) 35.3 against 35.0, the output head (429 MB) 71.0 against
-    // 72.1.
+    // 72.1; and earlier where rows at once leave too few bytes in flight
+    // (weights from HBM): 32,768 x 2816 (98 MB) 22.9 against 24.8, x 3072 (107
+    // MB) 24.1 against 40.5, 40,000 x 3072 31.6 against 44.0.
     const bool large = staged && a.rows >= rb_max * 8 * num_cus &&
-                       a.rows * nb * kQ8Bytes * NM > (512LL << 10) * num_cus;
+                       (a.rows * nb * kQ8Bytes * NM > (512LL << 10) * num_cus || nb > 80);
     // The other two kernels read a quantized activation; a graph capture that
     // finds no workspace for one can allocate none, and takes this one.
     const size_t sbytes = ((size_t)nb * sizeof(float) + 255) / 256 * 256;

@@ -258,6 +258,24 @@ def test_q8_0_matvecs_at_the_tiles_edges(ctx, rows, cols, shift):
     assert I.rel_err(gate[:rows], ref * orc_gelu(ref)) < 1e-5
 
 
+@pytest.mark.parametrize("rows", [32767, 32768, 32771])
+def test_q8_0_matvec_of_many_long_rows(ctx, rows):
+    """3072 columns on both sides of where rows are streamed: 512 rows of
+    weights repeated, so the oracle's 512 sums repeat too."""
+    cols, period = 3072, 512
+    w = I.q8_0_bytes(matrix(rows, period, cols))
+    d = dev(w).repeat(rows // period + 1)[: rows * cols // 32 * 34].contiguous()
+    x = np.random.default_rng(rows).standard_normal(cols).astype(np.float32)
+    xs, xq = q8_activation(ctx, x)
+    ref = np.resize(orc.matvec_q8_0(w, period, cols, host(xs), host(xq)), rows)
+    out = torch.full((rows + 1,), 7.0, device="cuda")
+    for run in (lambda: ctx.matvec_q8_0(d, rows, cols, xs, xq, out), lambda: ctx.project_q8_0(d, rows, cols, dev(x), out)):
+        out.fill_(7.0)
+        run()
+        got = host(out)
+        assert got[rows] == 7.0 and np.array_equal(got[:rows].view(np.uint32), ref.view(np.uint32))
+
+
 def orc_gelu(v):
     v = v.astype(np.float64)
     return 0.5 * v * (1.0 + np.tanh(0.7978846 * v * (1.0 + 0.044715 * v * v)))
