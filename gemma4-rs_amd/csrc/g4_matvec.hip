@@ -20,7 +20,8 @@
 // below the output head's size bring all their rows at once instead, with the
 // activation quantized once per workgroup (f32 activations, the engine's
 // comparison numerics, go the same way).  BF16 and F32 rows, one sum per
-// element, split the loading and the adding over two wavefronts.
+// element, split the loading and the adding over two wavefronts.  Many short
+// rows take a lane each, in every format.
 
 #include <algorithm>
 #include <type_traits>
@@ -702,6 +703,21 @@ __global__ __launch_bounds__(128) void matvec_dense_kernel(const W *__restrict__
     if (lane < n_rows) out[row0 + lane] = sum;
 }
 
+// The same, one lane per row: for many rows of a few values, of which the
+// kernel above uses one lane in eight or fewer.
+template <typename W>
+__global__ __launch_bounds__(256) void matvec_dense_narrow_kernel(const W *__restrict__ w, int64_t rows, int64_t cols,
+                                                                  const float *__restrict__ x,
+                                                                  float *__restrict__ out) {
+#pragma clang fp contract(off)
+    const int64_t row = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (row >= rows) return;
+    const W *r = w + row * cols;
+    float sum = -0.0f;
+    for (int64_t i = 0; i < cols; ++i) sum += weight_value(r[i]) * activation_value(W(), x[i]);
+    out[row] = sum;
+}
+
 template <int EPI, int NS>
 int launch_q8_rows(const MatvecArgs &a, int g, int rb, hipStream_t stream) {
     constexpr int NM = EPI >= kGeglu ? 2 : 1;
@@ -864,6 +880,22 @@ int launch_dense_rows(const MatvecArgs &a, hipStream_t stream) {
     return G4_OK;
 }
 
+// Short rows take a lane each where the two-wavefront kernel, whose time does
+// not fall with the columns below 256, would take longer, and the whole matrix
+// is small enough that the lanes' scattered reads hit a cache.  Measured (us,
+// lane per row / two wavefronts): bf16 off the 16-byte loads 2048 x 7 4 / 5,
+// 8192 x 33 5 / 6, 16,384 x 33 5 / 8, 32,768 x 50 7 / 12, 100,000 x 50 16 / 27, 200,000
+// x 33 18 / 51, 50,000 x 100 17 / 18; with them 16,384 x 32 6 / 5, 32,768 x 32 6 /
+// 8, 262,144 x 32 18 / 38; f32 off them 32,768 x 50 8 / 9, 100,000 x 50 (20 MB) 22
+// / 20, 200,000 x 39 (31 MB) 46 / 42; with them 500,000 x 32 (64 MB) 257 / 73.
+template <typename W>
+bool dense_lane_per_row(const MatvecArgs &a, bool vec, int64_t num_cus) {
+    const int64_t per_cu = a.rows / num_cus;
+    if (a.cols <= 0 || a.rows > (1LL << 30) || a.rows * a.cols * (int64_t)sizeof(W) > (32LL << 20)) return false;
+    if (a.cols <= 40) return per_cu >= (vec ? 128 : 64) || (!vec && a.cols <= 16);
+    return !vec && a.cols <= 64 && per_cu >= 128 && a.rows * a.cols * (int64_t)sizeof(W) <= (16LL << 20);
+}
+
 // Rows per workgroup of the BF16 / F32 mat-vecs.  Up to eight rows per CU
 // every wavefront has a SIMD of its own with 4 rows, and the shorter loads
 // start the chain sooner (1024 x 1536 bf16: 6.6 us against 7.2 with 16).
@@ -872,6 +904,12 @@ int launch_dense_rows(const MatvecArgs &a, hipStream_t stream) {
 template <typename W>
 int launch_dense(g4_ctx *ctx, const MatvecArgs &a, hipStream_t stream) {
     const bool vec = (uintptr_t)a.w % 4 == 0 && a.cols * sizeof(W) % 16 == 0 && a.cols < (1LL << 24);
+    if (dense_lane_per_row<W>(a, vec, ctx->num_cus)) {
+        hipLaunchKernelGGL(matvec_dense_narrow_kernel<W>, dim3((unsigned)((a.rows + 255) / 256)), dim3(256), 0, stream,
+                           (const W *)a.w, a.rows, a.cols, a.x, a.out);
+        G4_HIP(hipGetLastError());
+        return G4_OK;
+    }
     if (!vec) return launch_dense_rows<W, 4, 2, false>(a, stream);
     if (a.rows <= 8LL * ctx->num_cus) return launch_dense_rows<W, 4, 4, true>(a, stream);
     return launch_dense_rows<W, 16, 3, true>(a, stream);

@@ -149,7 +149,8 @@ def test_bf16_and_f32_matvecs_bit_exact(ctx, rows, cols):
 
 
 @pytest.mark.parametrize("rows,cols", [(1, 1), (3, 8), (4, 255), (5, 256), (15, 257), (16, 264), (2048, 520), (2049, 520),
-                                       (2065, 1032), (2064, 250), (6, 40000)])
+                                       (2065, 1032), (2064, 250), (6, 40000), (16383, 33), (16384, 33), (32767, 32), (32768, 32),
+                                       (32768, 64), (32800, 65), (700, 16), (700, 17)])
 @pytest.mark.parametrize("shift", [0, 1])
 def test_bf16_and_f32_matvecs_at_the_tiles_edges(ctx, rows, cols, shift):
     """Row and column counts around the workgroup's rows and chunks, matrices
