@@ -1376,6 +1376,7 @@ constexpr int kMinUnitTiles = 4;  // a split leaves no piece shorter (unless the
 // once more, over `slices` workgroups.  More pieces per block than the merge
 // kernel's registers hold cost it another pass per 16.
 constexpr double kMergePass = 0.5;
+constexpr double kLptFavour = 0.97;  // see build_schedule
 
 using Piece = std::array<int, 3>;  // block, t_lo, t_hi
 using BlockTiles = std::vector<std::pair<int, int>>;  // [t_lo, t_hi) per block
@@ -1523,6 +1524,10 @@ static bool stream_pack(const BlockTiles &bt, const std::vector<int> &seq, doubl
 // every chunk is a new shape, so this runs on the way to its first launch:
 // flat arrays and few candidates keep it at 0.04-0.2 ms (0.15-2 ms with nested
 // vectors, lengths in steps of 8 tiles and 12 capacities, at no better cost).
+// LPT cuts the blocks at about the same places, so that workgroups read the
+// same tiles at the same time; stream-K has to beat it by 3%.  (Without: 130
+// queries of 2 KV heads at position 6000, d = 512, 156 us, so 134; 228 shapes
+// 0.8% faster in the mean, the slowest against their best schedule 17% -> 5%.)
 static int build_schedule(const BlockTiles &bt, int n_bins, const ScheduleCost &sc, Bins &bins, int *slices) {
     int max_tiles = 1;
     long long total = 0;
@@ -1544,6 +1549,7 @@ static int build_schedule(const BlockTiles &bt, int n_bins, const ScheduleCost &
         lpt_pack(bt, ut, n_bins, sc, k);
         consider();
     }
+    best.cost *= kLptFavour;
     // Largest, smallest, second largest, second smallest, ...
     std::vector<int> order(bt.size()), seq;
     for (size_t i = 0; i < order.size(); ++i) order[i] = (int)i;
