@@ -324,7 +324,7 @@ __device__ inline void stage_activation(float *act, int nb, const float *xs, con
 // Weights from HBM, activation as f32 (one wavefront per two or three rows
 // that quantized the activation for itself, before -> here): 2048 x 1536
 // 5.4 -> 4.0 us, 4096 x 1536 6.3 -> 5.0, 1536 x 6144 11.3 -> 7.1, gate and up
-// of 6144 x 1536 (20.9 MB) 10.3 -> 7.6; a plain read of 16 MiB takes 4.7.
+// of 6144 x 1536 (20.1 MB) 10.3 -> 7.6; a plain read of 16 MiB takes 4.7.
 // f32 activations, one lane per row before: 2048 x 1536 27 -> 3.8 us,
 // 1536 x 6144 172 -> 7.0.
 template <int EPI, int DOT>
