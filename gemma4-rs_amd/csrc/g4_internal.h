@@ -61,7 +61,8 @@ namespace g4 {
 bool capturing(hipStream_t stream);
 
 // Grows the context's workspace to at least `bytes` (stream-ordered users
-// must not be in flight on another stream when it grows).
+// must not be in flight on another stream when it grows; a graph captured
+// over it keeps the buffer it was captured with).
 int ensure_workspace(g4_ctx *ctx, size_t bytes, hipStream_t stream);
 // Makes ctx->zero_rows hold at least n zero int64 values.
 int ensure_zero_rows(g4_ctx *ctx, int64_t n, hipStream_t stream);

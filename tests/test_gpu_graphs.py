@@ -193,8 +193,9 @@ def test_prepare_and_decode_step_in_a_graph(ctx):
 
 @pytest.mark.parametrize("rows,cols", [(4096, 1536), (70000, 1536)])
 def test_q8_0_matvecs_in_a_graph(ctx, rows, cols):
-    """Small matrices quantize inside the mat-vec; large ones quantize into
-    the context's workspace first (a second kernel in the graph)."""
+    """Most matrices quantize inside the mat-vec; the gate and up pair of
+    70,000 rows (228 MB) quantizes into the context's workspace first (a
+    second kernel in the graph)."""
     w = dev(I.q8_0_bytes(np.random.default_rng(rows).uniform(-1, 1, rows * cols).astype(np.float32)))
     up = dev(I.q8_0_bytes(np.random.default_rng(rows + 1).uniform(-1, 1, rows * cols).astype(np.float32)))
     x = torch.randn(cols, device="cuda")

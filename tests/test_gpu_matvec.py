@@ -72,7 +72,7 @@ SHAPES = [
     (1536, 6144),  # FFN down: 192 blocks a row
     (77, 512),
     (5, 8192),     # 256 blocks a row
-    (33, 96),      # cols not a multiple of 256: the row-per-lane kernel
+    (33, 96),      # cols not a multiple of 256
     (1, 32),
     (4099, 1536),  # rows not a multiple of the row tile
 ]
@@ -201,8 +201,8 @@ def test_shape_errors(ctx):
 def test_fused_quantization_entries_equal_the_two_step_calls(ctx, rows, cols):
     """project / gated FFN / logits with the activation quantized inside the
     call: bit for bit the quantize_q8_0 + mat-vec pair (model.rs:211-212,
-    236-237, 447).  An f32 activation that is not 16-byte aligned and column
-    counts outside the LDS-staged kernel take the two-step route inside."""
+    236-237, 447), also for an f32 activation that is not 16-byte aligned and
+    column counts that are not a multiple of 256."""
     gate = dev(I.q8_0_bytes(matrix(8, rows, cols)))
     up = dev(I.q8_0_bytes(matrix(9, rows, cols)))
     xh = np.random.default_rng(rows).standard_normal(cols + 1).astype(np.float32)

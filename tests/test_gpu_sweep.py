@@ -109,8 +109,10 @@ def test_ragged_decode_split_sizes(ctx, d, B, bound):
 
 @pytest.mark.parametrize("d,bound", [(256, 512), (512, 250), (256, 130)])
 def test_ragged_decode_after_non_finite_partials(ctx, d, bound):
-    """The merge reads split slots past a short sequence's count: left full
-    of NaN by an earlier batch, they must not reach its output."""
+    """The merge reads split slots past a short sequence's count: outputs
+    left full of NaN there by an earlier batch's V must not reach its own.
+    (Those batches' maxima and sums are finite; a test below poisons
+    them.)"""
     B = 6
     K = np.random.default_rng(d).standard_normal((B * bound, d), dtype=np.float32) * 0.1
     V = np.full((B * bound, d), np.nan, np.float32)
