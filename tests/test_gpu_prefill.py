@@ -132,6 +132,31 @@ def test_prefill_non_finite_scores_fail_the_call(ctx, d, window):
                            pos0, window)
 
 
+@pytest.mark.parametrize("d,window,pos0,N", [(512, 0, 3000, 24), (256, 4096, 6000, 20), (512, 0, 9000, 17)])
+def test_non_finite_values_where_workgroups_share_units(ctx, d, window, pos0, N):
+    """Few queries deep in a context, whose units leave many partials: a
+    non-finite V reaches only the queries that attend it; pieces whose every
+    score is -inf weigh nothing; a NaN score fails the call and leaves
+    nothing for the next."""
+    units = [f(pos0, N, window, d, 1, 256)[0] for f in (g4hip.prefill_schedule, g4hip.prefill_launch_schedule)]
+    assert len(units[1]) > len(units[0])
+    if N >= 24:
+        test_prefill_non_finite_v_reaches_only_the_queries_that_attend_it(ctx, d, window, pos0, N)
+    q, K, V = case(51 + d + pos0, pos0 + N, d, d == 512)
+    q = np.ascontiguousarray(q).copy()
+    q.reshape(pos0 + N, 8, d)[:, :, 3] = np.abs(q.reshape(pos0 + N, 8, d)[:, :, 3]) + 0.5
+    Kx = K.copy()
+    Kx[pos0 - 2500:pos0 - 300, 3] = -np.inf
+    got = prefill(ctx, q[pos0:], Kx, V, pos0, N, window, d)
+    check_all_rows(f"-inf pieces d={d}", got, q[pos0:], Kx, V, pos0, window)
+    Kx[pos0 - 200, 3] = np.nan
+    out = torch.zeros(N * 8 * d, device="cuda")
+    ctx.attend_prefill(dev(q[pos0:]), dev(Kx), dev(V), pos0, N, window, 8, 1, d, out)
+    with pytest.raises(g4hip.EngError, match="softmax input is not finite"):
+        ctx.check_status()
+    check_all_rows(f"after it d={d}", prefill(ctx, q[pos0:], K, V, pos0, N, window, d), q[pos0:], K, V, pos0, window)
+
+
 def test_prefill_never_reads_future_or_out_of_window_rows(ctx):
     """Rows after the chunk and before the first window hold NaN."""
     d, W, pos0, N = 256, 64, 200, 50

@@ -300,7 +300,7 @@ def test_attend_prefill_is_the_token_loop(n_heads, n_kv, d, pos0, N, window):
 @pytest.mark.parametrize("n_heads,n_kv,d,pos0,N,window", [(8, 1, 32, 200, 37, 0), (8, 1, 32, 130, 29, 100),
                                                         (4, 2, 16, 0, 70, 0), (8, 1, 16, 61, 9, 1)])
 def test_blocked_prefill_is_the_token_loop(n_heads, n_kv, d, pos0, N, window):
-    """or_attend_prefill_blocked (the checker's fast loop nest: groups of 4
+    """or_attend_prefill_blocked (the deep-context tests' fast loop nest: groups of 4
     queries walking 64-key chunks together) equals or_attend_prefill bit for
     bit -- outputs, statuses and the untouched heads of a failing query --
     on ranges that cross chunk and group edges, on any thread count."""
